@@ -100,6 +100,28 @@ static bool use_contig(const AxisGeom &g, int order, int hi_kind, bool f64) {
     return true;
 }
 
+// Shortest pencil of the constant-coefficient kernels (cssx_uniform.hpp): the corrections of the two
+// ends must not reach each other, a^(n-4) below the rounding of the type.
+static int uniform_min(bool f64) { return f64 ? 48 : 32; }
+
+// Whether a launch runs on the constant-coefficient kernels: walls at both ends (unit-stride pencils that
+// lie back to back, or strided ones) or the periodic wrap (strided), of enough rows, with nothing asked for
+// but f' (the assembled rows of compact_fd6 and its halo ends stay with the plan-driven kernels).
+static bool use_uniform(const DerivSpec *sp, int nspec, const AxisGeom &g, bool f64) {
+    if (g.n < uniform_min(f64) || g.n > 1024) return false;
+    const bool unit = g.srow == 1;
+    int M, G, S;
+    if (!unit && !seg_shape(g.n, f64, 0, M, G, S)) return false;
+    if (unit && (g.sa != g.n || (g.nb > 1 && g.sb != (long)g.n * g.na))) return false;
+    for (int i = 0; i < nspec; i++) {
+        const DerivSpec &s = sp[i];
+        const bool wall = s.lo_kind == END_WALL && s.hi_kind == END_WALL;
+        const bool wrap = s.lo_kind == END_PERIODIC && s.hi_kind == END_PERIODIC;
+        if (!(wall || (wrap && !unit)) || s.rhs_out || s.lo_r0_val || s.plan) return false;
+    }
+    return true;
+}
+
 static int lanes_per_pencil(int n, int MR) {
     const int nl = (n + MR - 1) / MR;
     int Lw = 1;
@@ -116,11 +138,17 @@ static void fill_launch_geom(DerivLaunch<T> &L, const AxisGeom &g) {
     L.njobs = 0;
 }
 
-// Kernel family of a batched launch: 2 = the wide kernel (long strided pencils, several
+// Kernel family of a batched launch: 4 / 3 = the constant-coefficient kernels (strided /
+// contiguous), 2 = the wide kernel (long strided pencils, several
 // segments per wavefront), 1 = the contiguous kernel, 0 = the strided kernel; seg = its rows
 // per segment (or per lane).  The wide and contiguous D2 upper-wall closures need the last
 // segment to own >= 2 rows.
 static void launch_family(const DerivSpec *sp, int nspec, const AxisGeom &g, bool f64, int &variant, int &seg) {
+    if (use_uniform(sp, nspec, g, f64)) {
+        variant = g.srow == 1 ? 3 : 4;
+        seg = g.n <= 512 ? 8 : 16;   // rows per lane of the contiguous kernel
+        return;
+    }
     int WM = 0, WG = 0;
     if (g.srow != 1) wide_shape(g.n, f64, WM, WG);
     bool wide = WM > 0;
@@ -151,7 +179,7 @@ static int add_job(DerivLaunch<T> &L, const DerivSpec *specs, int nspec, int i, 
     const DerivSpec &s = specs[i];
     const PlanKey key = launch_plan_key(specs, nspec, i, g, f64);
     const void *plan = s.plan;
-    if (!plan) {
+    if (!plan && key.variant < 3) {
         int rc = get_plan(key, f64 ? CSSX_PREC_F64 : CSSX_PREC_F32, &plan);
         if (rc) return rc;
     }
@@ -176,9 +204,10 @@ static int deriv_impl(const DerivSpec &sp, const AxisGeom &g, int nspec, hipStre
     const bool f64 = sizeof(T) == 8;
     int variant = 0, seg = 0;
     launch_family(&sp, nspec, g, f64, variant, seg);
-    const bool wide = variant == 2, contig = variant == 1;
+    const bool wide = variant == 2, contig = variant == 1, line = variant == 3;
     if (contig) { L.M = seg; L.S = lanes_per_pencil(g.n, L.M); }
-    for (int i = 0; i < nspec && !contig; i++)   // only the contiguous kernel writes end-row taps
+    if (line) { L.M = seg; L.S = (g.n + seg - 1) / seg; }
+    for (int i = 0; i < nspec && !contig && !line; i++)   // only the contiguous kernels write end-row taps
         if ((&sp)[i].tap_in || (&sp)[i].tap_out) return CSSX_EINVAL;
     if (wide) { L.M = seg; L.S = (g.n + seg - 1) / seg; }
     double passes = 0.0;
@@ -192,7 +221,9 @@ static int deriv_impl(const DerivSpec &sp, const AxisGeom &g, int nspec, hipStre
         if (L.njobs == kMaxJobs || i == nspec - 1) {
             const int phase = g.phase;
             const int tok = timing_begin(phase, stream);
-            hipError_t e = wide ? launch_deriv_wide<T>(L, s.order, stream)
+            hipError_t e = variant == 4 ? launch_deriv_seg<T>(L, s.order, stream)
+                           : line ? launch_deriv_line<T>(L, s.order, stream)
+                           : wide ? launch_deriv_wide<T>(L, s.order, stream)
                                 : contig ? launch_deriv_contig<T>(L, s.order, stream) : launch_deriv<T>(L, s.order, stream);
             timing_end(tok, stream, passes * g.n * (double)g.na * g.nb * sizeof(T));
             if (e != hipSuccess) return CSSX_EHIP;
@@ -257,6 +288,12 @@ extern "C" int cssx_ctx_create(const cssx_grid *grid, cssx_ctx **out) {
                     for (int bd = 0; bd < 5; bd++) {
                         if (ax == CSSX_AXIS_PHI && (lo == 0 || hi == 0)) continue;
                         if (lo == 1 && hi == 1 && bd > 0) continue;
+                        // walls at both ends: no plan where the constant-coefficient kernels serve both
+                        // precisions
+                        int sM, sG, sS;
+                        if (lo == 0 && hi == 0 && ns[ax] >= uniform_min(true) &&
+                            (ax == CSSX_AXIS_THETA || (seg_shape(ns[ax], true, 0, sM, sG, sS) && seg_shape(ns[ax], false, 0, sM, sG, sS))))
+                            continue;
                         PlanKey key{ns[ax], order, lo ? END_HALO : END_WALL, hi ? END_HALO : END_WALL, bd};
                         const void *p;
                         for (int var = 0; var < 2; var++) {
@@ -530,6 +567,7 @@ extern "C" int cssx_compact_fd6_noalloc(int n, long npencils, double dri, int ib
     double *ptr = nullptr;
     if ((rc = scratch_address(&ptr))) return rc;
     const PlanKey key = launch_plan_key(&s, 1, 0, g, true);
+    if (key.variant >= 3) return run_derivs(&s, 1, g, CSSX_PREC_F64, st);   // no plan table
     const std::vector<double> *plan = nullptr;
     {
         std::lock_guard<std::mutex> lk(g_scratch_mu);

@@ -51,6 +51,14 @@ template <typename T>
 hipError_t launch_deriv_contig(const DerivLaunch<T> &L, int order, hipStream_t stream);
 template <typename T>
 hipError_t launch_deriv_wide(const DerivLaunch<T> &L, int order, hipStream_t stream);
+// walls at both ends or the periodic wrap, pencils of at least 48 (FP64) / 32 (FP32) rows
+template <typename T>
+hipError_t launch_deriv_seg(const DerivLaunch<T> &L, int order, hipStream_t stream);
+// the segmentation of that kernel for a launch of `cols` columns; false: n has none
+bool seg_shape(int n, bool f64, long cols, int &M, int &G, int &S);
+// walls at both ends, unit row stride, same lengths (L.M rows per lane, L.S lanes per pencil)
+template <typename T>
+hipError_t launch_deriv_line(const DerivLaunch<T> &L, int order, hipStream_t stream);
 // (M, G) of the wide strided kernel for a pencil of n rows (M = 0: k_deriv serves it)
 void wide_shape(int n, bool f64, int &M, int &G);
 

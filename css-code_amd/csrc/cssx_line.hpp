@@ -1,0 +1,173 @@
+// One pencil along the lanes of a wavefront: loads, the constant-coefficient compact solve
+// (cssx_uniform.hpp) and stores of a unit-stride pencil whose lane j holds rows [j*MR, j*MR + MR).
+// Several pencils sit side by side in a wavefront; lanes past the last pencil take part with zeros.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "cssx_bufio.hpp"
+#include "cssx_uniform.hpp"
+
+namespace cssx {
+
+// n and nl are wave-uniform, so kn2, m and every comparison with a row number k below are scalar; with
+// FULL (n a multiple of MR) they are compile-time.
+template <int MR, bool FULL>
+struct LineShape {
+    int n, nl, j, m;      // pencil rows, lanes per pencil, this lane, rows of the last lane
+    int jn2, kn2;         // lane and position of row n-2
+    bool active, first, last, at_n2;
+    __device__ __forceinline__ LineShape(int n_, int nl_, int j_, bool act)
+        : n(n_), nl(nl_), j(j_), m(FULL ? MR : n_ - (nl_ - 1) * MR), jn2(FULL ? nl_ - 1 : (n_ - 2) / MR),
+          kn2(FULL ? MR - 2 : (n_ - 2) % MR), active(act), first(act && j_ == 0), last(act && j_ == nl_ - 1),
+          at_n2(act && j_ == (FULL ? nl_ - 1 : (n_ - 2) / MR)) {}
+    template <typename T>
+    __device__ __forceinline__ T pick(const T (&v)[MR], int k0) const {
+        T r = v[MR - 1];
+#pragma unroll
+        for (int k = 0; k < MR - 1; k++) {
+            const T t = v[k];   // (read first: a conditional read would index the array in scratch)
+            r = k == k0 ? t : r;
+        }
+        return r;
+    }
+};
+
+// MR values at p + at as 16-byte loads (4-byte alignment); a lane whose run leaves the `total` values
+// there (the last lane of the last pencil) reads them one by one.  Rows past the pencil's end belong to the
+// next pencil: the caller's rows beyond n-1 are not used.
+template <typename T, int MR, bool FULL>
+__device__ __forceinline__ void line_load(const T *__restrict__ p, long at, long total, const LineShape<MR, FULL> &G,
+                                          T (&v)[MR]) {
+#pragma unroll
+    for (int k = 0; k < MR; k++) v[k] = T(0);
+    if (!G.active) return;
+    if (FULL || at + MR <= total) {
+        __builtin_memcpy(v, p + at, sizeof(v));
+    } else {
+#pragma unroll
+        for (int k = 0; k < MR; k++)
+            if (at + k < total) v[k] = p[at + k];
+    }
+}
+
+template <typename T, int MR, bool FULL>
+__device__ __forceinline__ void line_store(T *__restrict__ p, long at, const LineShape<MR, FULL> &G, const T (&x)[MR]) {
+    if (FULL || !G.last || G.m == MR) {
+        __builtin_memcpy(p + at, x, sizeof(x));
+    } else {
+#pragma unroll
+        for (int k = 0; k < MR; k++)
+            if (k < G.m) p[at + k] = x[k];
+    }
+}
+
+// The derivative of the wavefront's pencils (walls at both ends), times `scale`, in x; row n-1 comes back
+// as the return value of the lane that holds row n-2 (see line_last).  lo_val / hi_val: the prescribed
+// wall derivatives in index units, read on the lanes of rows 0 and n-2.  v's rows past n-1 are
+// overwritten.
+template <typename T, int ORDER, int MR, bool FULL>
+__device__ __forceinline__ T line_solve(const LineShape<MR, FULL> &G, T (&v)[MR], int bd, T lo_val, T hi_val, T scale,
+                                        T (&x)[MR]) {
+    using U = Uni<ORDER>;
+    // carries that reach `reach` rows span this many lanes
+    constexpr int NT = (uni_reach<T, ORDER>() + MR - 1) / MR;
+    constexpr T A = (T)U::a, Q = (T)uni_pow<ORDER>(MR);
+    const int kn2 = G.kn2;
+    // window: rows -4 .. MR+1 of the lane (two rows on either side for the stencil, two more below
+    // for the upper closure)
+    T lo[4], hi[2];
+#pragma unroll
+    for (int k = 0; k < 4; k++) lo[k] = from_prev(v[MR - 4 + k]);
+    hi[0] = from_next(v[0]);
+    hi[1] = from_next(v[1]);
+    auto f = [&](int k) -> T { return k < 0 ? lo[k + 4] : k < MR ? v[k] : hi[k - MR]; };
+    // ---- wall rows
+    T r0 = T(0), r1 = T(0), q0 = T(0), q1 = T(0);
+    {
+        const T e[6] = {v[0], v[1], v[2], v[3], v[4], v[5]};
+        wall_rhs<T, ORDER, false>(e, bd, lo_val, false, scale, r0, r1);
+    }
+#pragma unroll
+    for (int k = 0; k < MR; k++)
+        if (k == kn2) {
+            const T e[6] = {f(k + 1), f(k), f(k - 1), f(k - 2), f(k - 3), f(k - 4)};
+            wall_rhs<T, ORDER, true>(e, bd, hi_val, false, scale, q0, q1);
+        }
+    // ---- forward: rows 0, 1 and n-2, n-1 are not uniform rows and stay zero
+    const Stencil<T, ORDER> S(scale);
+    T y[MR], p = T(0);
+#pragma unroll
+    for (int k = 0; k < MR; k++) {
+        T t = S(f(k - 2), f(k - 1), v[k], f(k + 1), f(k + 2)) - A * p;
+        if (k < 2) t = G.j == 0 ? T(0) : t;
+        y[k] = p = t;
+    }
+    // the carry out of a lane: its last row (lanes that hold row n-2 or follow it send nothing)
+    const bool up = G.active && G.j < G.jn2;
+    T Z = T(0);
+#pragma unroll
+    for (int i = 0; i < NT; i++) Z = from_prev(up ? y[MR - 1] + Q * Z : T(0));
+    // (rows 0, 1 of the lower wall stay zero: lane 0 receives no carry)
+#pragma unroll
+    for (int k = 0; k < MR && k < uni_reach<T, ORDER>(); k++) y[k] += (T)uni_pow<ORDER>(k + 1) * Z;
+    // ---- upper wall: row n-2 from y of row n-3, which starts the backward recurrence
+    const bool dhi = bd == 1 || bd == 2, dlo = bd == 1 || bd == 3;
+    const T yprev = FULL ? T(0) : from_prev(y[MR - 1]);
+    T xn1 = T(0);
+#pragma unroll
+    for (int k = 0; k < MR; k++)
+        if (k == kn2) {
+            T xn2;
+            upper_wall<T, ORDER>(k > 0 ? y[k > 0 ? k - 1 : 0] : yprev, q0, q1, dhi, xn2, xn1);
+            y[k] = G.at_n2 ? xn2 : y[k];
+        } else if (k > kn2) {
+            y[k] = G.j >= G.jn2 ? T(0) : y[k];
+        }
+    if (!FULL && G.j > G.jn2) {
+#pragma unroll
+        for (int k = 0; k < MR; k++) y[k] = T(0);
+    }
+    // ---- backward
+    T xp = T(0);
+#pragma unroll
+    for (int k = MR - 1; k >= 0; k--) {
+        xp = y[k] - A * xp;
+        x[k] = xp;
+    }
+    const bool dn = G.active && G.j > 0;
+    const T xf = x[0];
+    Z = T(0);
+#pragma unroll
+    for (int i = 0; i < NT; i++) Z = from_next(dn ? xf + Q * Z : T(0));
+#pragma unroll
+    for (int k = MR - 1; k >= 0 && MR - k <= uni_reach<T, ORDER>(); k--) x[k] += (T)uni_pow<ORDER>(MR - k) * Z;
+    // ---- lower wall: rows 0, 1 and the correction of the rows above, passed up the lanes
+    T x0, x1;
+    T c = lower_wall<T, ORDER>(x[2], r0, r1, dlo, x0, x1) * (T)uni_pow<ORDER>(-2);
+    c = G.first ? c : T(0);
+    T cs = c;
+#pragma unroll
+    for (int i = 1; i < NT; i++) {
+        c = from_prev(up ? c : T(0)) * Q;
+        cs += c;
+    }
+#pragma unroll
+    for (int k = 0; k < MR; k++) x[k] += (T)uni_pow<ORDER>(k) * cs;
+    x[0] = G.first ? x0 : x[0];
+    x[1] = G.first ? x1 : x[1];
+    return xn1;
+}
+
+// puts row n-1 (returned by line_solve on row n-2's lane) in its place
+template <typename T, int MR, bool FULL>
+__device__ __forceinline__ void line_last(const LineShape<MR, FULL> &G, T xn1, T (&x)[MR]) {
+#pragma unroll
+    for (int k = 0; k < MR - 1; k++)
+        if (k == G.kn2) x[k + 1] = G.at_n2 ? xn1 : x[k + 1];
+    if (G.kn2 == MR - 1) {
+        const T t = from_prev(G.at_n2 ? xn1 : T(0));
+        x[0] = (G.active && G.j == G.jn2 + 1) ? t : x[0];
+    }
+}
+
+}  // namespace cssx
