@@ -11,6 +11,8 @@
 //                       GELU' (backward), split-K atomic accumulation (weight gradients)
 //   * k_mse, k_colsum, k_adam   loss gradient, bias gradients, Adam (FP32 master weights,
 //                       BF16 copies for the matrix cores)
+//   * k_train_*         the same training step of a 128-wide network in three launches
+//                       (cssx_train.hpp)
 //   * k_add_closure     un-standardized network output -> the FP32 tendency that the RHS adds
 //
 // Every matrix here is row-major.  A layer is Z = X W + b, H = GELU(Z), with W stored as
@@ -614,6 +616,10 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
     }
 }
 
+}  // namespace cssx
+#include "cssx_train.hpp"
+namespace cssx {
+
 inline unsigned nblk(long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
 }  // namespace cssx
@@ -632,6 +638,10 @@ struct cssx_mlp {
     float *Z1 = nullptr, *Z2 = nullptr, *Y = nullptr, *dY = nullptr, *dZ2 = nullptr, *dZ1 = nullptr, *loss = nullptr;
     cssx_bf16 *H1 = nullptr, *H2 = nullptr, *dYb = nullptr, *dZ2b = nullptr, *dZ1b = nullptr, *X = nullptr;
     float *xmean = nullptr, *xistd = nullptr, *ymean = nullptr, *ystd = nullptr;
+    // fused training step (h1 = h2 = 128): transposed BF16 weights, partial weight gradients, and per
+    // workgroup of 32 rows the bias sums and squared error
+    cssx_bf16 *WT = nullptr;
+    float *part = nullptr, *wgbias = nullptr, *wgloss = nullptr;
     cssx_bf16 *pk = nullptr;        // weights packed for the fused inference kernel (h1 = h2 = 128)
     long step = 0;
     void *blk = nullptr;
@@ -676,6 +686,48 @@ int mlp_forward(cssx_mlp *n, const cssx_bf16 *X, int rows, bool keep_z, hipStrea
     g = ga(n->H2, n->h2, 1, n->Wb + n->oW3, n->nout, 1, rows, n->nout, n->h2, EPI_STORE);
     g.bias = n->W + n->ob3; g.C = n->Y; g.ldc = n->nout;
     return gemm(g, 1, s);
+}
+
+// the BF16 copies of the FP32 weights
+void weight_copies(cssx_mlp *n) {
+    if (n->WT)
+        hipLaunchKernelGGL(k_train_copies, dim3(nblk(n->np)), dim3(256), 0, 0, n->W, n->np, n->oW2, n->oW3, n->Wb, n->WT);
+    else
+        hipLaunchKernelGGL(k_to_bf16, dim3(nblk(n->np)), dim3(256), 0, 0, n->W, n->Wb, n->np);
+}
+
+// Whether the three-launch gradient serves these rows: its network, and 16-byte aligned feature rows (a row
+// is 27 16-byte units).
+bool train_fused(const cssx_mlp *n, const void *X) { return n->WT && (reinterpret_cast<uintptr_t>(X) & 15) == 0; }
+
+// The loss gradient (adam null) or a whole Adam step in three launches (cssx_train.hpp).
+int mlp_train(cssx_mlp *n, const cssx_bf16 *X, const float *Tg, int rows, float *loss, const AdamArgs *adam, hipStream_t s) {
+    const int nwg = (rows + kTrRows - 1) / kTrRows;
+    TrainBufs o;
+    o.XT = n->X; o.H1T = n->H1; o.H2T = n->H2; o.dYT = n->dYb; o.dZ2T = n->dZ2b; o.dZ1T = n->dZ1b;
+    o.ld = (long)nwg * kTrRows;
+    o.bias = n->wgbias;
+    o.loss = n->wgloss;
+    hipLaunchKernelGGL(k_train_rows, dim3(nwg), dim3(512), 0, s, X, Tg, rows, (const cssx_bf16 *)n->WT,
+                       (const cssx_bf16 *)(n->Wb + n->oW2), (const cssx_bf16 *)(n->Wb + n->oW3), (const float *)(n->W + n->ob1),
+                       (const float *)(n->W + n->ob2), (const float *)(n->W + n->ob3), o);
+    // splits of at least 256 rows (8 products of 32 per wavefront tile): 8192 rows fill 1536 wavefronts
+    int chunk = 256;
+    while ((o.ld + chunk - 1) / chunk > kTrSplit) chunk *= 2;
+    const int splits = (int)((o.ld + chunk - 1) / chunk);
+    hipLaunchKernelGGL(k_train_wgrad, dim3(kTrWaveTiles / 4, splits), dim3(256), 0, s, o, rows, chunk, n->oW2, n->oW3, n->np,
+                       n->part);
+    const int nw = (int)nblk(n->np), nb = (kTrBias + 31) / 32 + 1;
+    const float cnt = (float)((long)rows * n->nout);
+    if (adam)
+        hipLaunchKernelGGL(k_train_apply<true>, dim3(nw + nb), dim3(256), 0, s, (const float *)n->part, splits, n->np, n->ob1,
+                           n->oW2, n->ob2, n->oW3, n->ob3, (const float *)n->wgbias, (const float *)n->wgloss, nwg, cnt, nw,
+                           n->G, n->loss, loss, *adam);
+    else
+        hipLaunchKernelGGL(k_train_apply<false>, dim3(nw + nb), dim3(256), 0, s, (const float *)n->part, splits, n->np, n->ob1,
+                           n->oW2, n->ob2, n->oW3, n->ob3, (const float *)n->wgbias, (const float *)n->wgloss, nwg, cnt, nw,
+                           n->G, n->loss, loss, AdamArgs{});
+    return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
 
 // gradients of the mean squared error of the last forward into n->G (zeroed first)
@@ -818,11 +870,13 @@ extern "C" int cssx_mlp_create(int nin, int h1, int h2, int nout, int max_rows, 
     n->nin = nin; n->h1 = h1; n->h2 = h2; n->nout = nout; n->max_rows = max_rows;
     n->oW1 = 0; n->ob1 = n->oW1 + (long)nin * h1; n->oW2 = n->ob1 + h1; n->ob2 = n->oW2 + (long)h1 * h2;
     n->oW3 = n->ob2 + h2; n->ob3 = n->oW3 + (long)h2 * nout; n->np = n->ob3 + nout;
-    const long R = max_rows;
-    const long fl = 4 * n->np + R * (2L * h1 + 2L * h2 + 2L * nout) + 1 + 2L * nin + 2L * nout;
-    const long bf = n->np + R * (h1 + h2 + nout + h2 + h1 + nin);
+    const bool fused = h1 == kTrH && h2 == kTrH;
+    const long R = ((long)max_rows + kTrRows - 1) / kTrRows * kTrRows, nwg = R / kTrRows;
+    const long fl = 4 * n->np + R * (2L * h1 + 2L * h2 + 2L * nout) + 1 + 2L * nin + 2L * nout +
+                    (fused ? kTrSplit * n->np + nwg * (kTrBias + 1) : 0);
+    const long bf = n->np + R * (h1 + h2 + nout + h2 + h1 + nin) + kTrWT;
     char *p = nullptr;
-    const size_t bytes = (size_t)fl * 4 + (size_t)bf * 2 + kPackBytes + 64 * 16;
+    const size_t bytes = (size_t)fl * 4 + (size_t)bf * 2 + kPackBytes + 32 * 256;
     if (hipMalloc((void **)&p, bytes) != hipSuccess) {
         delete n;
         return CSSX_ENOMEM;
@@ -837,6 +891,12 @@ extern "C" int cssx_mlp_create(int nin, int h1, int h2, int nout, int max_rows, 
     n->Wb = takeb(n->np); n->H1 = takeb(R * h1); n->H2 = takeb(R * h2); n->dYb = takeb(R * nout);
     n->dZ2b = takeb(R * h2); n->dZ1b = takeb(R * h1); n->X = takeb(R * nin);
     n->pk = takeb((long)(kPackBytes / 2));
+    if (fused) {
+        n->WT = takeb(kTrWT);
+        n->part = takef(kTrSplit * n->np);
+        n->wgbias = takef(nwg * kTrBias);
+        n->wgloss = takef(nwg);
+    }
     // PyTorch-Linear-style initialization: U(-1/sqrt(fan_in), 1/sqrt(fan_in)) for W and b
     std::vector<float> w(n->np), zeros(n->np, 0.0f), ones(nin, 1.0f);
     uint64_t s = seed;
@@ -856,7 +916,7 @@ extern "C" int cssx_mlp_create(int nin, int h1, int h2, int nout, int max_rows, 
               hipMemcpy(n->ymean, zo.data(), nout * 4, hipMemcpyHostToDevice) == hipSuccess &&
               hipMemcpy(n->ystd, oo.data(), nout * 4, hipMemcpyHostToDevice) == hipSuccess;
     if (ok) {
-        hipLaunchKernelGGL(k_to_bf16, dim3(nblk(n->np)), dim3(256), 0, 0, n->W, n->Wb, n->np);
+        weight_copies(n);
         ok = hipDeviceSynchronize() == hipSuccess;
     }
     if (!ok) {
@@ -880,7 +940,7 @@ extern "C" long cssx_mlp_num_params(const cssx_mlp *n) { return n ? n->np : -1; 
 extern "C" int cssx_mlp_set_params(cssx_mlp *n, const float *host_params) {
     if (!n || !host_params) return CSSX_EINVAL;
     if (hipMemcpy(n->W, host_params, n->np * 4, hipMemcpyHostToDevice) != hipSuccess) return CSSX_EHIP;
-    hipLaunchKernelGGL(k_to_bf16, dim3(nblk(n->np)), dim3(256), 0, 0, n->W, n->Wb, n->np);
+    weight_copies(n);
     return hipDeviceSynchronize() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
 
@@ -922,6 +982,7 @@ extern "C" int cssx_mlp_grad(cssx_mlp *n, const void *x_bf16, const float *targe
                              void *stream) {
     if (!n || !x_bf16 || !target || rows < 1 || rows > n->max_rows) return CSSX_EINVAL;
     hipStream_t s = (hipStream_t)stream;
+    if (train_fused(n, x_bf16)) return mlp_train(n, (const cssx_bf16 *)x_bf16, target, rows, loss, nullptr, s);
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, s, n->loss, 1L, 0.0f);
     int rc = mlp_forward(n, (const cssx_bf16 *)x_bf16, rows, true, s);
     if (!rc) rc = mlp_backward(n, (const cssx_bf16 *)x_bf16, target, rows, s);
@@ -932,13 +993,22 @@ extern "C" int cssx_mlp_grad(cssx_mlp *n, const void *x_bf16, const float *targe
 
 extern "C" int cssx_mlp_train_step(cssx_mlp *n, const void *x_bf16, const float *target, int rows, float lr,
                                    float *loss, void *stream) {
-    int rc = cssx_mlp_grad(n, x_bf16, target, rows, loss, stream);
+    if (!n || !x_bf16 || !target || rows < 1 || rows > n->max_rows) return CSSX_EINVAL;
+    const bool fused = train_fused(n, x_bf16);
+    int rc = fused ? CSSX_OK : cssx_mlp_grad(n, x_bf16, target, rows, loss, stream);
     if (rc) return rc;
     n->step++;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = (float)(1.0 - std::pow(0.9, (double)n->step)), c2 = (float)(1.0 - std::pow(0.999, (double)n->step));
+    if (fused) {
+        const AdamArgs A{n->W, n->Mo, n->Vo, n->Wb, n->WT, lr, b1, b2, 1e-8f, c1, c2};
+        return mlp_train(n, (const cssx_bf16 *)x_bf16, target, rows, loss, &A, (hipStream_t)stream);
+    }
     hipLaunchKernelGGL(k_adam, dim3(nblk(n->np)), dim3(256), 0, (hipStream_t)stream, n->W, n->G, n->Mo, n->Vo, n->Wb,
                        n->np, lr, b1, b2, 1e-8f, c1, c2);
+    if (n->WT)   // unaligned rows of a 128-wide network: keep the transposed copy in step
+        hipLaunchKernelGGL(k_train_copies, dim3(nblk(n->np)), dim3(256), 0, (hipStream_t)stream, n->W, n->np, n->oW2, n->oW3,
+                           n->Wb, n->WT);
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
 
