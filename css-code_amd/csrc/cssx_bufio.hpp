@@ -56,6 +56,15 @@ __device__ __forceinline__ T from_prev(T v) { return dpp_shift<0x138>(v); }
 template <typename T>
 __device__ __forceinline__ T from_next(T v) { return dpp_shift<0x130>(v); }
 
+// Workgroups are dealt to the 8 XCDs (and their L2s) round-robin.  The index that makes runs of 16
+// consecutive workgroups of one XCD neighbours in memory: where rows are no whole cache lines, two neighbours
+// write parts of the same line, which merge in one L2 but not across two.  Groups of 128; the last,
+// incomplete one is left as it is.
+__device__ __forceinline__ unsigned xcd_neighbour(unsigned i, unsigned n) {
+    const unsigned g = i & ~127u, r = i & 127u;
+    return g + 128u <= n ? g + (r & 7u) * 16u + (r >> 3) : i;
+}
+
 // v from lane l of the wavefront as a wave-uniform value (v_readlane)
 __device__ __forceinline__ float lane_val(float v, int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));

@@ -111,7 +111,7 @@ static bool use_uniform(const DerivSpec *sp, int nspec, const AxisGeom &g, bool 
     if (g.n < uniform_min(f64) || g.n > 1024) return false;
     const bool unit = g.srow == 1;
     int M, G, S;
-    if (!unit && !seg_shape(g.n, f64, 0, M, G, S)) return false;
+    if (!unit && !seg_shape(g.n, f64, 0, 1, M, G, S)) return false;
     if (unit && (g.sa != g.n || (g.nb > 1 && g.sb != (long)g.n * g.na))) return false;
     for (int i = 0; i < nspec; i++) {
         const DerivSpec &s = sp[i];
@@ -292,7 +292,7 @@ extern "C" int cssx_ctx_create(const cssx_grid *grid, cssx_ctx **out) {
                         // precisions
                         int sM, sG, sS;
                         if (lo == 0 && hi == 0 && ns[ax] >= uniform_min(true) &&
-                            (ax == CSSX_AXIS_THETA || (seg_shape(ns[ax], true, 0, sM, sG, sS) && seg_shape(ns[ax], false, 0, sM, sG, sS))))
+                            (ax == CSSX_AXIS_THETA || (seg_shape(ns[ax], true, 0, 1, sM, sG, sS) && seg_shape(ns[ax], false, 0, 1, sM, sG, sS))))
                             continue;
                         PlanKey key{ns[ax], order, lo ? END_HALO : END_WALL, hi ? END_HALO : END_WALL, bd};
                         const void *p;

@@ -26,6 +26,7 @@ struct SegArgs {
     int S, base, rem;      // segments; rows of a segment: base + 1 in the first rem, base in the others
     T q0, q1;              // (-a)^base, (-a)^(base+1)
     T up0, up1;            // (-a)^(base-M), (-a)^(base+1-M)
+    int near_xcd;          // neighbouring columns on one XCD (xcd_neighbour)
 };
 
 // EVEN: every segment has M rows (n = S*M), which takes the tests on a segment's last rows out.
@@ -51,7 +52,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(G == 1 ? 8
     const bool edge = wv == 0 || (wv + 1) * G >= S;
     const bool wall = J.lo_kind == END_WALL;             // both ends, or the periodic wrap
     // column c of the launch: pencil (a, b); addresses relative to the block's first b
-    const unsigned cols = (unsigned)L.na * (unsigned)L.nb, c0 = blockIdx.x * P;
+    const unsigned cols = (unsigned)L.na * (unsigned)L.nb, c0 = (A.near_xcd ? xcd_neighbour(blockIdx.x, gridDim.x) : blockIdx.x) * P;
     const bool pen_ok = c0 + p < cols;
     const bool active = pen_ok && seg_ok;
     unsigned a = c0 + (pen_ok ? p : 0), b = 0, b0 = 0;
@@ -303,11 +304,14 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(G == 1 ? 8
 
 // (M, G, S) of a pencil of n rows: S segments whose lengths ceil(n/S) and floor(n/S) both lie in
 // (M-4, M] of an instantiated M, G per wavefront.  Segments of up to 32 (FP32) / 16 (FP64) rows, the
-// most a lane holds without spilling, re-read the fewest halo rows; a launch of `cols` columns that would
-// leave wavefront slots empty with them (8192 on the chip) takes segments of up to 16, then 8 rows, whose
-// shorter chains end sooner (right-hand side of 64x64x128 points in FP32: 113 us with 32-row, 101 with 16-row
-// and 97 with 8-row segments; at 128x128x128 16-row segments measured best).  False if n has none.
-bool seg_shape(int n, bool f64, long cols, int &M, int &G, int &S) {
+// most a lane holds without spilling, re-read the fewest halo rows and serve fields that come from memory;
+// for fields that stay in the L2s shorter chains end sooner.  FP32, one field, 32- against 16- against
+// 8-row segments: 128x256x512 27.0, 30.7, 33.2 us; 97x203x331 (26 MB) 16.6, 18.3, 20.9; 90x151x250 (14 MB) 10.8,
+// 9.4, 11.9; right-hand side of 64x64x128 points (2 MB a field, up to 6 a launch) 113, 101, 97; FP64 there 139
+// (16) and 135 (8).  False if n has none.
+bool seg_shape(int n, bool f64, long cols, int njobs, int &M, int &G, int &S) {
+    const double mb = (double)n * (double)cols * (f64 ? 8.0 : 4.0) / 1e6;
+    const int want = njobs > 1 && mb <= 4.5 ? 8 : f64 || mb <= 16.0 ? 16 : 32;
     bool found = false;
     for (int most = f64 ? 16 : 32; most >= 8; most /= 2) {
         const int g = n <= 16 * most ? 1 : n <= 32 * most ? 2 : 4;
@@ -325,7 +329,7 @@ bool seg_shape(int n, bool f64, long cols, int &M, int &G, int &S) {
                 break;
             }
         }
-        if (found && (cols + 63) / 64 * S >= 8192) break;
+        if (found && most <= want) break;
     }
     return found;
 }
@@ -334,7 +338,7 @@ template <typename T>
 hipError_t launch_deriv_seg(const DerivLaunch<T> &L0, int order, hipStream_t stream) {
     DerivLaunch<T> L = L0;
     int M, G, S;
-    if (!seg_shape(L.n, sizeof(T) == 8, (long)L.na * L.nb * L.njobs, M, G, S) || L.njobs < 1 || L.njobs > kMaxJobs || L.n < 32)
+    if (!seg_shape(L.n, sizeof(T) == 8, (long)L.na * L.nb, L.njobs, M, G, S) || L.njobs < 1 || L.njobs > kMaxJobs || L.n < 32)
         return hipErrorInvalidValue;
     // 32-bit byte offsets of a lane: columns of up to 64 / na + 2 slow indices
     const int P = 64 / G;
@@ -369,6 +373,12 @@ hipError_t launch_deriv_seg(const DerivLaunch<T> &L0, int order, hipStream_t str
     const long cols = (long)L.na * L.nb;
     const dim3 grid((unsigned)((cols + P - 1) / P), L.njobs), block(64 * ((S + G - 1) / G));
     const bool even = L.n == S * M;
+    // Neighbouring columns on one XCD: in launches of more workgroups than the chip holds several times over
+    // (256x512x1024 FP32 phi 224 -> 201 us, r 217 -> 215; ragged 311x333x411 r 109 -> 90), and on phi also in
+    // smaller ones whose rows are no whole lines (97x203x331 20.6 -> 18.7).  Small r sweeps, whose rows lie
+    // whole planes apart, lost by it (97x203x331 16.6 -> 19.5).
+    const bool lines = ((long)L.na * sizeof(T)) % 128 == 0;
+    A.near_xcd = grid.x > 2048 || (L.nb > 1 && !lines);
 #define CSSX_LAUNCH_S(MM, GG)                                                                                     \
     do {                                                                                                          \
         if (even) {                                                                                               \

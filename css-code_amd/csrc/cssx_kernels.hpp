@@ -54,8 +54,8 @@ hipError_t launch_deriv_wide(const DerivLaunch<T> &L, int order, hipStream_t str
 // walls at both ends or the periodic wrap, pencils of at least 48 (FP64) / 32 (FP32) rows
 template <typename T>
 hipError_t launch_deriv_seg(const DerivLaunch<T> &L, int order, hipStream_t stream);
-// the segmentation of that kernel for a launch of `cols` columns; false: n has none
-bool seg_shape(int n, bool f64, long cols, int &M, int &G, int &S);
+// the segmentation of that kernel for a launch of njobs fields of `cols` columns; false: n has none
+bool seg_shape(int n, bool f64, long cols, int njobs, int &M, int &G, int &S);
 // walls at both ends, unit row stride, same lengths (L.M rows per lane, L.S lanes per pencil)
 template <typename T>
 hipError_t launch_deriv_line(const DerivLaunch<T> &L, int order, hipStream_t stream);

@@ -4,22 +4,35 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "cssx_bufio.hpp"
 #include "cssx_uniform.hpp"
 
 namespace cssx {
 
-// n and nl are wave-uniform, so kn2, m and every comparison with a row number k below are scalar; with
-// FULL (n a multiple of MR) they are compile-time.
-template <int MR, bool FULL>
+// REM = n mod MR, which makes the last lane's row count m and the place kn2 of row n-2 compile-time; -1: known
+// at run time only (n and nl are wave-uniform, so the comparisons with a row number k below are scalar).
+template <int MR, int REM>
 struct LineShape {
+    static constexpr bool FULL = REM == 0;   // every lane holds MR rows
     int n, nl, j, m;      // pencil rows, lanes per pencil, this lane, rows of the last lane
     int jn2, kn2;         // lane and position of row n-2
     bool active, first, last, at_n2;
-    __device__ __forceinline__ LineShape(int n_, int nl_, int j_, bool act)
-        : n(n_), nl(nl_), j(j_), m(FULL ? MR : n_ - (nl_ - 1) * MR), jn2(FULL ? nl_ - 1 : (n_ - 2) / MR),
-          kn2(FULL ? MR - 2 : (n_ - 2) % MR), active(act), first(act && j_ == 0), last(act && j_ == nl_ - 1),
-          at_n2(act && j_ == (FULL ? nl_ - 1 : (n_ - 2) / MR)) {}
+    __device__ __forceinline__ LineShape(int n_, int nl_, int j_, bool act) : n(n_), nl(nl_), j(j_), active(act) {
+        if constexpr (REM >= 0) {
+            m = REM == 0 ? MR : REM;
+            kn2 = (REM + MR - 2) % MR;
+            jn2 = REM == 1 ? nl - 2 : nl - 1;
+        } else {
+            m = n - (nl - 1) * MR;
+            kn2 = (n - 2) % MR;
+            jn2 = (n - 2) / MR;
+        }
+        first = act && j == 0;
+        last = act && j == nl - 1;
+        at_n2 = act && j == jn2;
+    }
     template <typename T>
     __device__ __forceinline__ T pick(const T (&v)[MR], int k0) const {
         T r = v[MR - 1];
@@ -35,13 +48,13 @@ struct LineShape {
 // MR values at p + at as 16-byte loads (4-byte alignment); a lane whose run leaves the `total` values
 // there (the last lane of the last pencil) reads them one by one.  Rows past the pencil's end belong to the
 // next pencil: the caller's rows beyond n-1 are not used.
-template <typename T, int MR, bool FULL>
-__device__ __forceinline__ void line_load(const T *__restrict__ p, long at, long total, const LineShape<MR, FULL> &G,
+template <typename T, int MR, int REM>
+__device__ __forceinline__ void line_load(const T *__restrict__ p, long at, long total, const LineShape<MR, REM> &G,
                                           T (&v)[MR]) {
 #pragma unroll
     for (int k = 0; k < MR; k++) v[k] = T(0);
     if (!G.active) return;
-    if (FULL || at + MR <= total) {
+    if (REM == 0 || at + MR <= total) {
         __builtin_memcpy(v, p + at, sizeof(v));
     } else {
 #pragma unroll
@@ -50,23 +63,34 @@ __device__ __forceinline__ void line_load(const T *__restrict__ p, long at, long
     }
 }
 
-template <typename T, int MR, bool FULL>
-__device__ __forceinline__ void line_store(T *__restrict__ p, long at, const LineShape<MR, FULL> &G, const T (&x)[MR]) {
-    if (FULL || !G.last || G.m == MR) {
+template <typename T, int MR, int REM>
+__device__ __forceinline__ void line_store(T *__restrict__ p, long at, const LineShape<MR, REM> &G, const T (&x)[MR]) {
+    if (REM == 0 || !G.last || G.m == MR) {
         __builtin_memcpy(p + at, x, sizeof(x));
-    } else {
-#pragma unroll
-        for (int k = 0; k < MR; k++)
-            if (k < G.m) p[at + k] = x[k];
+        return;
     }
+    // the last lane's m < MR rows in pieces of 8, 4, 2 and 1 (m is wave-uniform; one store per set bit)
+    auto piece = [&](auto cnt, int from) {
+        constexpr int C = decltype(cnt)::value;
+#pragma unroll
+        for (int f = 0; f + C <= MR; f += C)
+            if (f == from) __builtin_memcpy(p + at + f, &x[f], C * sizeof(T));
+    };
+    int from = 0;
+    if constexpr (MR > 8) {
+        if (G.m & 8) piece(std::integral_constant<int, 8>{}, from), from += 8;
+    }
+    if (G.m & 4) piece(std::integral_constant<int, 4>{}, from), from += 4;
+    if (G.m & 2) piece(std::integral_constant<int, 2>{}, from), from += 2;
+    if (G.m & 1) piece(std::integral_constant<int, 1>{}, from);
 }
 
 // The derivative of the wavefront's pencils (walls at both ends), times `scale`, in x; row n-1 comes back
 // as the return value of the lane that holds row n-2 (see line_last).  lo_val / hi_val: the prescribed
 // wall derivatives in index units, read on the lanes of rows 0 and n-2.  v's rows past n-1 are
 // overwritten.
-template <typename T, int ORDER, int MR, bool FULL>
-__device__ __forceinline__ T line_solve(const LineShape<MR, FULL> &G, T (&v)[MR], int bd, T lo_val, T hi_val, T scale,
+template <typename T, int ORDER, int MR, int REM>
+__device__ __forceinline__ T line_solve(const LineShape<MR, REM> &G, T (&v)[MR], int bd, T lo_val, T hi_val, T scale,
                                         T (&x)[MR]) {
     using U = Uni<ORDER>;
     // carries that reach `reach` rows span this many lanes
@@ -112,7 +136,8 @@ __device__ __forceinline__ T line_solve(const LineShape<MR, FULL> &G, T (&v)[MR]
     for (int k = 0; k < MR && k < uni_reach<T, ORDER>(); k++) y[k] += (T)uni_pow<ORDER>(k + 1) * Z;
     // ---- upper wall: row n-2 from y of row n-3, which starts the backward recurrence
     const bool dhi = bd == 1 || bd == 2, dlo = bd == 1 || bd == 3;
-    const T yprev = FULL ? T(0) : from_prev(y[MR - 1]);
+    // (needed where row n-2 may sit first in its lane)
+    const T yprev = (REM < 0 || REM == 2) ? from_prev(y[MR - 1]) : T(0);
     T xn1 = T(0);
 #pragma unroll
     for (int k = 0; k < MR; k++)
@@ -123,7 +148,7 @@ __device__ __forceinline__ T line_solve(const LineShape<MR, FULL> &G, T (&v)[MR]
         } else if (k > kn2) {
             y[k] = G.j >= G.jn2 ? T(0) : y[k];
         }
-    if (!FULL && G.j > G.jn2) {
+    if ((REM < 0 || REM == 1) && G.j > G.jn2) {
 #pragma unroll
         for (int k = 0; k < MR; k++) y[k] = T(0);
     }
@@ -159,8 +184,8 @@ __device__ __forceinline__ T line_solve(const LineShape<MR, FULL> &G, T (&v)[MR]
 }
 
 // puts row n-1 (returned by line_solve on row n-2's lane) in its place
-template <typename T, int MR, bool FULL>
-__device__ __forceinline__ void line_last(const LineShape<MR, FULL> &G, T xn1, T (&x)[MR]) {
+template <typename T, int MR, int REM>
+__device__ __forceinline__ void line_last(const LineShape<MR, REM> &G, T xn1, T (&x)[MR]) {
 #pragma unroll
     for (int k = 0; k < MR - 1; k++)
         if (k == G.kn2) x[k + 1] = G.at_n2 ? xn1 : x[k + 1];
