@@ -3,19 +3,18 @@
 // faces (the Dbydr/Dbydt/Dbydp closures of derivatives.f90:547-796, :1010-1262 applied on
 // every axis, as Determine_Dtype's dtype 0 would ask); all three first derivatives of every
 // patch are work items of one kernel:
-//   * r and phi (strided) items: a workgroup of NT lanes covers P = NT/SM pencils cut
-//     into SM >= ceil(n/M) segments of M rows (lane = segment * P + pencil), loads stay
-//     coalesced along theta, the segment solves run in registers and the interface system by
-//     parallel cyclic reduction over SM lanes (the contiguous-kernel plan cut at M); each
-//     strided job takes M or M2 rows per segment, whichever wastes fewer lanes;
-//   * theta (contiguous) items: lanes walk the pencil in runs of MR rows (the contiguous
-//     kernel's scheme) with the halo rows exchanged by DPP wave shifts.
-// Workgroups loop over the item table (persistent, as many as can be resident), staging each
-// item's plan in LDS.  (M, M2, MR, NT) are template choices; cssx_patchset_autotune times the
-// instantiated variants on the actual patch set.
+//   * r and phi items (seg_item): a workgroup of NT lanes covers P = NT/S columns cut into S segments (a power
+//     of two) of M-4 .. M rows, lane = segment * P + column, the columns numbered over both pencil indices;
+//   * theta items (line_item): every wavefront walks whole pencils in runs of MR rows per lane;
+// both with the constant-coefficient recurrences of cssx_uniform.hpp: an item reads no plan, a seg_item
+// exchanges its carries at two barriers and a line_item has none.  Pencils too short for them (fewer than
+// 32 rows in FP32, 48 in FP64) run on the plan-driven strided_item / contig_item.
+// Workgroups loop over the item table (persistent, as many as can be resident).  (MR, NT) are template
+// choices; cssx_patchset_autotune times the instantiated variants on the actual patch set.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 #include <map>
 #include <new>
 #include <tuple>
@@ -25,6 +24,7 @@
 #include "cssx_bufio.hpp"
 #include "cssx_internal.hpp"
 #include "cssx_kernels.hpp"
+#include "cssx_line.hpp"
 #include "cssx_plan.hpp"
 #include "cssx_rows.hpp"
 
@@ -38,8 +38,13 @@ struct PatchJob {
     int n, na, nb, lanes;   // pencil length, pencils (a fast, b slow), SM or lanes per pencil
     long sa, sb, srow;
     T scale;
-    int bdry, kind;         // kind 0 strided (M rows per segment), 2 strided (M2), 1 contiguous
+    int bdry, kind;         // 0 strided and 1 contiguous (plan-driven), 2 segments, 3 lines
+    // kind 2: columns are na x nb flattened (nb = 1 where they lie back to back); S segments of base + 1 (the
+    // first rem) or base rows, P = 2^lgp columns per item, and the powers of -a of those lengths
+    int S, lgp, M, base, rem;
+    T q0, q1, up0, up1;
 };
+enum PatchKind { PK_STRIDED = 0, PK_CONTIG = 1, PK_SEG = 2, PK_LINE = 3 };
 
 constexpr int kPatchTail = 3 * kMaxLanes + 2 * kPcrSteps * kMaxLanes;
 // capacity of each padded interface exchange array: SM*(P+1) or P*(SM+1) = NT + max(SM, P)
@@ -281,38 +286,209 @@ __device__ __forceinline__ void contig_item(const PatchJob<T> &J, int ablk, int 
     __syncthreads();   // LDS reused by the next item
 }
 
-// FP32 with runs of 8 rows fits 64 VGPRs: eight waves per SIMD (two 1024-lane or four 512-lane
-// workgroups per CU); the other variants would spill there
-template <typename T, int M, int M2, int MR, int NT>
+// S segments of the columns [blk*P, +P) (the recurrences and exchanges of k_deriv_seg)
+template <typename T, int M, int NT>
+__device__ __forceinline__ void seg_item(const PatchJob<T> &J, int blk, T *sp) {
+    using U = Uni<1>;
+    constexpr int TAIL = 5, REACH = uni_reach<T, 1>(), NTERM = (REACH + M - TAIL) / (M - TAIL + 1);
+    constexpr T a_ = (T)U::a;
+    T *sh_y = sp, *sh_x = sp + NT, *sh_lo = sp + 2 * NT;   // sh_lo: two values per column
+    const int tid = threadIdx.x, n = J.n, S = J.S, P = 1 << J.lgp;
+    const int k = tid >> J.lgp, p = tid & (P - 1);
+    const int st = k * J.base + min(k, J.rem), m = J.base + (k < J.rem ? 1 : 0);
+    const bool lo = k == 0, hi = k == S - 1;
+    const unsigned cols = (unsigned)J.na * (unsigned)J.nb, c = (unsigned)blk * P + p;
+    unsigned a = c, b = 0;
+    if (J.nb > 1) {
+        b = c / (unsigned)J.na;
+        a = c - b * (unsigned)J.na;
+    }
+    const unsigned rowb = (unsigned)J.srow * (unsigned)sizeof(T);
+    // the resource spans the patch: loads of lanes without a column read zero, their stores are dropped
+    const unsigned span = (unsigned)n * (unsigned)J.na * (unsigned)J.nb * (unsigned)sizeof(T);
+    const unsigned lofs = c < cols ? (a * (unsigned)J.sa + b * (unsigned)J.sb) * (unsigned)sizeof(T) : kNoPencil;
+    const __amdgpu_buffer_rsrc_t rin = span_rsrc(J.in, span);
+    // w[i] = row st - 2 + i; past a wall any row of the pencil will do
+    T w[M + 4];
+    const unsigned v0 = lofs + (unsigned)st * rowb;
+    {
+        const int dlo = lo ? 2 : 0;
+#pragma unroll
+        for (int i = 0; i < M + 4; i++) {
+            if (i < 2) w[i] = bload<T>(rin, lofs + (unsigned)(st - 2 + i + dlo) * rowb, 0u);
+            else if (i >= M - TAIL + 3) w[i] = bload<T>(rin, lofs + (unsigned)min(st - 2 + i, n - 1) * rowb, 0u);
+            else w[i] = bload<T>(rin, v0, (unsigned)(i - 2) * rowb);
+        }
+    }
+    const T scale = J.scale;
+    const int bd = J.bdry;
+    T r0 = T(0), r1 = T(0), q0 = T(0), q1 = T(0);
+    if (lo) {
+        const T e[6] = {w[2], w[3], w[4], w[5], w[6], w[7]};
+        wall_rhs<T, 1, false>(e, bd, T(0), false, scale, r0, r1);
+    }
+    if (hi) {
+        T e[6];   // row n-1 sits at w[m + 1]
+#pragma unroll
+        for (int t = 0; t < 6; t++) {
+            e[t] = w[M + 1 - t];
+#pragma unroll
+            for (int s = 1; s < TAIL; s++) e[t] = m == M - s ? w[M + 1 - t - s] : e[t];
+        }
+        wall_rhs<T, 1, true>(e, bd, T(0), false, scale, q0, q1);
+    }
+    const Stencil<T, 1> St(scale);
+    const int me = hi ? m - 2 : m;
+    T y[M], yp = T(0), yl = T(0);
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+        T t = St(w[j], w[j + 1], w[j + 2], w[j + 3], w[j + 4]) - a_ * yp;
+        if (j < 2) t = lo ? T(0) : t;
+        if (j > M - TAIL - 3) t = j < me ? t : T(0);
+        y[j] = yp = t;
+        if (j >= M - TAIL - 2) yl = j < me ? t : yl;
+    }
+    sh_y[tid] = yl;
+    __syncthreads();
+    auto qseg = [&](int s) -> T { return s < J.rem ? J.q1 : J.q0; };
+    T Y = T(0);
+#pragma unroll
+    for (int t = NTERM; t >= 1; t--)
+        if (k - t >= 0) Y = sh_y[(k - t) * P + p] + qseg(k - t) * Y;
+#pragma unroll
+    for (int j = 0; j < M && j < REACH + 2; j++) {
+        const T t = y[j] + (T)uni_pow<1>(j + 1) * Y;
+        y[j] = j > M - TAIL - 3 ? (j < me ? t : y[j]) : t;
+    }
+    T xn1 = T(0);
+    if (hi) {
+        T y3 = y[M - 3], xn2;
+#pragma unroll
+        for (int s = 1; s < TAIL; s++) y3 = m == M - s ? y[M - 3 - s] : y3;
+        upper_wall<T, 1>(y3, q0, q1, bd == 1 || bd == 2, xn2, xn1);
+#pragma unroll
+        for (int s = 0; s < TAIL; s++) y[M - 2 - s] = m == M - s ? xn2 : y[M - 2 - s];
+    }
+    T xp = T(0);
+#pragma unroll
+    for (int j = M - 1; j >= 0; j--) {
+        xp = y[j] - a_ * xp;
+        y[j] = xp;
+    }
+    sh_x[tid] = y[0];
+    if (lo) {
+        sh_lo[p] = y[2];
+        sh_lo[P + p] = r1 - (T)U::l1 * r0;
+    }
+    __syncthreads();
+    auto carry_x = [&](int kk) -> T {
+        T X = T(0);
+#pragma unroll
+        for (int t = NTERM; t >= 1; t--)
+            if (kk + t < S) X = sh_x[(kk + t) * P + p] + qseg(kk + t) * X;
+        return X;
+    };
+    {
+        const T X = carry_x(k) * (k < J.rem ? J.up1 : J.up0);
+#pragma unroll
+        for (int j = M - 1; j >= 0 && M - j <= REACH + TAIL; j--) y[j] += (T)uni_pow<1>(M - j) * X;
+    }
+    T x0 = T(0), x1 = T(0);
+    if (k <= (NTERM == 1 ? 0 : NTERM)) {
+        const T x2 = sh_lo[p] + (T)uni_pow<1>(-2) * (qseg(0) * carry_x(0));
+        T s = lower_wall<T, 1>(x2, T(0), sh_lo[P + p], bd == 1 || bd == 3, x0, x1) * (T)uni_pow<1>(-2);
+        if constexpr (NTERM > 1) {
+            T f = T(1);
+            for (int t = 0; t < k; t++) f *= qseg(t);
+            s *= f;
+        }
+#pragma unroll
+        for (int j = 0; j < M && j < REACH + 2; j++) y[j] += (T)uni_pow<1>(j) * s;
+        if (lo) {
+            y[0] = x0 + r0;
+            y[1] = x1;
+        }
+    }
+    if (hi) {
+#pragma unroll
+        for (int s = 0; s < TAIL; s++) y[M - 1 - s] = m == M - s ? xn1 : y[M - 1 - s];
+    }
+    const __amdgpu_buffer_rsrc_t rout = span_rsrc(J.out, span);
+#pragma unroll
+    for (int j = 0; j < M; j++)
+        if (j < M - TAIL + 1 || j < m) bstore(y[j], rout, v0, (unsigned)j * rowb);
+}
+
+// whole theta pencils [blk * pencils per workgroup, ...): every wavefront on its own
+template <typename T, int MR, int NT>
+__device__ __forceinline__ void line_item(const PatchJob<T> &J, int blk) {
+    const int n = J.n, nl = J.lanes, ppw = 64 / nl;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int pl = (int)((unsigned)lane * (unsigned)J.lgp >> 16), j = lane - pl * nl;   // lgp: ceil(2^16 / nl)
+    const unsigned np = (unsigned)J.na * (unsigned)J.nb, id0 = ((unsigned)blk * (NT / 64) + wv) * ppw;
+    if (id0 >= np) return;
+    const bool active = pl < ppw && id0 + pl < np;
+    const long at0 = (long)id0 * n, total = (long)np * n - at0;
+    const unsigned at = active ? (unsigned)(pl * n + j * MR) : 0u;
+    LineShape<MR, -1> G(n, nl, j, active);
+    T v[MR], x[MR];
+    line_load<T, MR>(J.in + at0, at, total, G, v);
+    const T xn1 = line_solve<T, 1, MR>(G, v, J.bdry, T(0), T(0), J.scale, x);
+    line_last<T, MR>(G, xn1, x);
+    if (active) line_store<T, MR>(J.out + at0, at, G, x);
+}
+
+// FP32 is held to 64 VGPRs: eight waves per SIMD (two 1024-lane or four 512-lane workgroups per CU)
+template <typename T, int MR, int NT>
 __global__ __launch_bounds__(NT, (sizeof(T) == 4 && MR == 8) ? 8 : 1) void k_patch_derivs(const PatchJob<T> *__restrict__ jobs,
                                                        const int4 *__restrict__ items, int nitems) {
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __align__(16) unsigned char smem_raw[];
     T *sp = reinterpret_cast<T *>(smem_raw);
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
-        const int4 w = items[it];
-        const PatchJob<T> J = jobs[w.x];
-        if (J.kind == 0) strided_item<T, M, NT>(J, w.y, w.z, sp);
-        else if (M2 != M && J.kind == 2) strided_item<T, M2, NT>(J, w.y, w.z, sp);
-        else contig_item<T, MR, NT>(J, w.y, w.z, sp);
+        const int4 w = items[xcd_neighbour(it, nitems)];
+        const PatchJob<T> &J = jobs[w.x];
+        if (J.kind == PK_LINE) {
+            line_item<T, MR, NT>(J, w.y);
+        } else if (J.kind == PK_SEG) {
+            if constexpr (sizeof(T) == 4) {
+                switch (J.M) {
+                case 20: seg_item<T, 20, NT>(J, w.y, sp); break;
+                case 24: seg_item<T, 24, NT>(J, w.y, sp); break;
+                case 28: seg_item<T, 28, NT>(J, w.y, sp); break;
+                default: seg_item<T, 32, NT>(J, w.y, sp); break;
+                }
+            } else {
+                if (J.M == 12) seg_item<T, 12, NT>(J, w.y, sp);
+                else seg_item<T, 16, NT>(J, w.y, sp);
+            }
+        } else if (J.kind == PK_STRIDED) {
+            __syncthreads();   // a seg_item before it may still be reading its exchange arrays
+            strided_item<T, 16, NT>(J, w.y, w.z, sp);
+        } else {
+            __syncthreads();
+            contig_item<T, 8, NT>(J, w.y, w.z, sp);
+        }
     }
 }
 
-// LDS bytes an item of pencil length n needs (the larger of the two schemes)
-inline size_t patch_lds(int nmax, int M, int MR, int NT, size_t elem) {
-    const int nl = (nmax + M - 1) / M;   // M: the shorter segment length in use
-    const size_t a = (size_t)5 * (nmax + nl) + 4 * (size_t)patch_shared(NT) + kPatchTail;
-    const size_t b = (size_t)5 * MR * ((nmax + MR - 1) / MR) + kPatchTail;
-    return std::max(a, b) * elem;
+// rows from which a patch axis runs on the constant-coefficient items
+template <typename T>
+constexpr int patch_uniform_min() { return sizeof(T) == 4 ? 32 : 48; }
+
+// LDS bytes: the exchange arrays of a seg_item, and the plan-driven items' for their longest pencil
+inline size_t patch_lds(int nmax_short, int NT, size_t elem) {
+    const size_t seg = (size_t)4 * NT;
+    if (nmax_short == 0) return seg * elem;
+    const int nl = (nmax_short + 15) / 16;
+    const size_t a = (size_t)5 * (nmax_short + nl) + 4 * (size_t)patch_shared(NT) + kPatchTail;
+    const size_t b = (size_t)5 * 8 * ((nmax_short + 7) / 8) + kPatchTail;
+    return std::max({seg, a, b}) * elem;
 }
 
-// the variants the autotuner chooses from: strided segment lengths (M, M2: each strided job
-// takes the one that wastes fewer lanes to the power-of-two segment count), contiguous run
-// length MR and workgroup size
+// the variants the autotuner chooses from: rows per lane of the theta items and workgroup size
 constexpr int kPatchVariants = 4;
-constexpr int kVarM[kPatchVariants] = {16, 16, 16, 16};
-constexpr int kVarM2[kPatchVariants] = {12, 16, 12, 12};
-constexpr int kVarMR[kPatchVariants] = {8, 8, 16, 8};
-constexpr int kVarNT[kPatchVariants] = {1024, 1024, 1024, 512};
+constexpr int kVarMR[kPatchVariants] = {8, 8, 16, 16};
+constexpr int kVarNT[kPatchVariants] = {1024, 512, 1024, 512};
 
 // ---- synthetic patch data: N(0,1) (SplitMix64 + Box-Muller, the generator of cssx/model.py's
 //      normal()) smoothed by [1,2,1]/4 along each axis with the edge value repeated --------------
@@ -387,7 +563,7 @@ extern "C" int cssx_patch_fill(void *out, void *tmp, int prec, int nr, int nth, 
 }
 
 struct cssx_patchset {
-    int prec = 0, npatch = 0, nmax = 0, best = 0;
+    int prec = 0, npatch = 0, nmax_short = 0, best = 0;   // nmax_short: longest plan-driven pencil
     long nitems[kPatchVariants] = {};
     void *jobs[kPatchVariants] = {};
     int4 *items[kPatchVariants] = {};
@@ -403,15 +579,15 @@ unsigned next_pow2(unsigned v) {
 
 template <typename T>
 int build_variant(cssx_patchset *ps, const cssx_patch *pt, int var) {
-    const int M = kVarM[var], M2 = kVarM2[var], MR = kVarMR[var], NT = kVarNT[var];
-    // lanes a strided job of n rows and na pencils per plane occupies with segments of m rows
-    auto strided_cost = [&](int n, long na, int m) {
-        const long sm = (long)next_pow2((unsigned)((n + m - 1) / m)), p = NT / sm;
-        return (na + p - 1) / p * (long)NT * m;
-    };
+    const int MR = kVarMR[var], NT = kVarNT[var];
     std::vector<PatchJob<T>> jobs;
     std::vector<int4> items;
     const int prec = sizeof(T) == 8 ? CSSX_PREC_F64 : CSSX_PREC_F32;
+    auto pw = [](int k) {
+        double v = 1.0;
+        for (int i = 0; i < std::abs(k); i++) v *= -Uni<1>::a;
+        return (T)(k < 0 ? 1.0 / v : v);
+    };
     for (int i = 0; i < ps->npatch; i++) {
         const cssx_patch &q = pt[i];
         const long sth = 1, sph = q.nth, sr = (long)q.nth * q.nphi;
@@ -425,53 +601,73 @@ int build_variant(cssx_patchset *ps, const cssx_patch *pt, int var) {
             if (ax == 0) { J.n = q.nr; J.na = q.nth; J.nb = q.nphi; J.sa = sth; J.sb = sph; J.srow = sr; J.scale = (T)q.dri; }
             else if (ax == 1) { J.n = q.nth; J.na = q.nphi; J.nb = q.nr; J.sa = sph; J.sb = sr; J.srow = sth; J.scale = (T)q.dti; }
             else { J.n = q.nphi; J.na = q.nth; J.nb = q.nr; J.sa = sth; J.sb = sr; J.srow = sph; J.scale = (T)q.dpi; }
-            J.kind = ax == 1 ? 1 : 0;
-            const int Mj = (J.kind == 0 && strided_cost(J.n, J.na, M2) < strided_cost(J.n, J.na, M)) ? M2 : M;
-            if (Mj != M) J.kind = 2;
+            const bool uniform = J.n >= patch_uniform_min<T>();
+            J.kind = ax == 1 ? (uniform ? PK_LINE : PK_CONTIG) : (uniform ? PK_SEG : PK_STRIDED);
             // the kernels' buffer ranges (span_rsrc): offsets up to kNoPencil + (n + 20) rows
             // stay below 2^32, and contiguous items walk unit-stride rows
-            if (J.kind != 1 && (double)(J.n + 20) * (double)J.srow * sizeof(T) > 2147483648.0) return CSSX_EINVAL;
-            if (J.kind == 1 && (J.srow != 1 || (double)J.na * (double)J.sa * sizeof(T) > 2147483648.0))
-                return CSSX_EINVAL;
-            PlanKey key{J.n, 1, END_WALL, END_WALL, q.bdry};
-            key.variant = J.kind == 1 ? 1 : 2;
-            key.seg = J.kind == 1 ? MR : Mj;
-            const void *plan = nullptr;
-            int rc = get_plan(key, prec, &plan);
-            if (rc) return rc;
-            J.plan = (const T *)plan;
+            if (ax != 1 && (double)(J.n + 20) * (double)J.srow * sizeof(T) > 2147483648.0) return CSSX_EINVAL;
+            if (ax == 1 && (J.srow != 1 || (double)J.na * (double)J.sa * sizeof(T) > 2147483648.0)) return CSSX_EINVAL;
             long per_b;
-            if (J.kind != 1) {
-                J.lanes = (int)next_pow2((unsigned)((J.n + Mj - 1) / Mj));
-                per_b = (J.na + (NT / J.lanes) - 1) / (NT / J.lanes);
+            int nb = J.nb;
+            if (J.kind == PK_SEG) {
+                // 32-row (FP32) or 16-row (FP64) segments at most, a power of two of them (a patch is at
+                // most 2^30 bytes: the resource of its columns fits)
+                const int most = sizeof(T) == 4 ? 32 : 16;
+                J.S = (int)next_pow2((unsigned)((J.n + most - 1) / most));
+                J.base = J.n / J.S;
+                J.rem = J.n % J.S;
+                J.M = (J.base + (J.rem > 0) + 3) / 4 * 4;
+                J.lgp = 0;
+                while ((J.S << (J.lgp + 1)) <= NT) J.lgp++;
+                J.q0 = pw(J.base); J.q1 = pw(J.base + 1);
+                J.up0 = pw(J.base - J.M); J.up1 = pw(J.base + 1 - J.M);
+                if (J.sb == J.na) {   // r: the two pencil indices are one contiguous run
+                    J.na *= J.nb;
+                    J.nb = 1;
+                }
+                nb = 1;
+                per_b = ((long)J.na * J.nb + (1 << J.lgp) - 1) >> J.lgp;
+            } else if (J.kind == PK_LINE) {
+                J.lanes = (J.n + MR - 1) / MR;
+                J.lgp = (65536 + J.lanes - 1) / J.lanes;
+                nb = 1;
+                const long pw_ = (long)(NT / 64) * (64 / J.lanes);
+                per_b = ((long)J.na * J.nb + pw_ - 1) / pw_;
             } else {
-                J.lanes = (int)next_pow2((unsigned)((J.n + MR - 1) / MR));
-                const int ppw = 64 / J.lanes;
-                const long pw = (long)(NT / 64) * ppw;
-                per_b = (J.na + pw - 1) / pw;
+                PlanKey key{J.n, 1, END_WALL, END_WALL, q.bdry};
+                key.variant = J.kind == PK_CONTIG ? 1 : 2;
+                key.seg = J.kind == PK_CONTIG ? 8 : 16;
+                const void *plan = nullptr;
+                int rc = get_plan(key, prec, &plan);
+                if (rc) return rc;
+                J.plan = (const T *)plan;
+                J.lanes = (int)next_pow2((unsigned)((J.n + key.seg - 1) / key.seg));
+                const long p = J.kind == PK_CONTIG ? (long)(NT / 64) * (64 / J.lanes) : NT / J.lanes;
+                per_b = (J.na + p - 1) / p;
+                ps->nmax_short = std::max(ps->nmax_short, J.n);
             }
             const int jid = (int)jobs.size();
             jobs.push_back(J);
-            for (int b = 0; b < J.nb; b++)
+            for (int b = 0; b < nb; b++)
                 for (long x = 0; x < per_b; x++) items.push_back(make_int4(jid, (int)x, b, 0));
         }
     }
     if (items.size() > (size_t)INT32_MAX) return CSSX_EINVAL;
     ps->nitems[var] = (long)items.size();
-    if (hipMalloc(&ps->jobs[var], jobs.size() * sizeof(PatchJob<T>)) != hipSuccess ||
+    if (hipMalloc(&ps->jobs[var], std::max<size_t>(1, jobs.size()) * sizeof(PatchJob<T>)) != hipSuccess ||
         hipMalloc((void **)&ps->items[var], std::max<size_t>(1, items.size()) * sizeof(int4)) != hipSuccess)
         return CSSX_ENOMEM;
-    if (hipMemcpy(ps->jobs[var], jobs.data(), jobs.size() * sizeof(PatchJob<T>), hipMemcpyHostToDevice) != hipSuccess ||
+    if ((jobs.size() && hipMemcpy(ps->jobs[var], jobs.data(), jobs.size() * sizeof(PatchJob<T>), hipMemcpyHostToDevice) != hipSuccess) ||
         (items.size() && hipMemcpy(ps->items[var], items.data(), items.size() * sizeof(int4),
                                    hipMemcpyHostToDevice) != hipSuccess))
         return CSSX_EHIP;
     return CSSX_OK;
 }
 
-template <typename T, int M, int M2, int MR, int NT>
+template <typename T, int MR, int NT>
 hipError_t launch_variant(const cssx_patchset *ps, int var, hipStream_t s) {
-    const size_t shm = patch_lds(ps->nmax, std::min(M, M2), MR, NT, sizeof(T));
-    const void *fn = (const void *)k_patch_derivs<T, M, M2, MR, NT>;
+    const size_t shm = patch_lds(ps->nmax_short, NT, sizeof(T));
+    const void *fn = (const void *)k_patch_derivs<T, MR, NT>;
     if (shm > 65536) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
@@ -485,7 +681,7 @@ hipError_t launch_variant(const cssx_patchset *ps, int var, hipStream_t s) {
     if (e != hipSuccess) return e;
     const long g = std::min<long>(ps->nitems[var], (long)ncu * std::max(1, per_cu));
     if (g < 1) return hipSuccess;
-    hipLaunchKernelGGL((k_patch_derivs<T, M, M2, MR, NT>), dim3((unsigned)g), dim3(NT), shm, s,
+    hipLaunchKernelGGL((k_patch_derivs<T, MR, NT>), dim3((unsigned)g), dim3(NT), shm, s,
                        (const PatchJob<T> *)ps->jobs[var], (const int4 *)ps->items[var], (int)ps->nitems[var]);
     return hipGetLastError();
 }
@@ -493,10 +689,10 @@ hipError_t launch_variant(const cssx_patchset *ps, int var, hipStream_t s) {
 template <typename T>
 hipError_t launch_any(const cssx_patchset *ps, int var, hipStream_t s) {
     switch (var) {
-    case 0: return launch_variant<T, 16, 12, 8, 1024>(ps, var, s);
-    case 1: return launch_variant<T, 16, 16, 8, 1024>(ps, var, s);
-    case 2: return launch_variant<T, 16, 12, 16, 1024>(ps, var, s);
-    default: return launch_variant<T, 16, 12, 8, 512>(ps, var, s);
+    case 0: return launch_variant<T, 8, 1024>(ps, var, s);
+    case 1: return launch_variant<T, 8, 512>(ps, var, s);
+    case 2: return launch_variant<T, 16, 1024>(ps, var, s);
+    default: return launch_variant<T, 16, 512>(ps, var, s);
     }
 }
 
@@ -515,7 +711,6 @@ extern "C" void cssx_patchset_destroy(cssx_patchset *ps) {
 extern "C" int cssx_patchset_create(const cssx_patch *patches, int npatch, int prec, cssx_patchset **out) {
     if (!patches || npatch < 1 || !out || (prec != CSSX_PREC_F64 && prec != CSSX_PREC_F32)) return CSSX_EINVAL;
     *out = nullptr;
-    int nmax = 0;
     for (int i = 0; i < npatch; i++) {
         const cssx_patch &q = patches[i];
         if (!q.in || q.nr < 8 || q.nth < 8 || q.nphi < 8 || q.nr > 512 || q.nth > 512 || q.nphi > 512 || q.bdry < 0 ||
@@ -523,13 +718,11 @@ extern "C" int cssx_patchset_create(const cssx_patch *patches, int npatch, int p
             return CSSX_EINVAL;
         const double bytes = (double)q.nr * q.nth * q.nphi * (prec == CSSX_PREC_F64 ? 8.0 : 4.0);
         if (bytes >= 4294967295.0) return CSSX_EINVAL;   // 32-bit buffer offsets
-        nmax = std::max({nmax, q.nr, q.nth, q.nphi});
     }
     cssx_patchset *ps = new (std::nothrow) cssx_patchset;
     if (!ps) return CSSX_ENOMEM;
     ps->prec = prec;
     ps->npatch = npatch;
-    ps->nmax = nmax;
     for (int v = 0; v < kPatchVariants; v++) {
         int rc = prec == CSSX_PREC_F64 ? build_variant<double>(ps, patches, v) : build_variant<float>(ps, patches, v);
         if (rc) {
