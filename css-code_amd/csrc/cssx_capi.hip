@@ -104,15 +104,15 @@ static bool use_contig(const AxisGeom &g, int order, int hi_kind, bool f64) {
 // ends must not reach each other, a^(n-4) below the rounding of the type.
 static int uniform_min(bool f64) { return f64 ? 48 : 32; }
 
-// Whether a launch runs on the constant-coefficient kernels: walls at both ends (unit-stride pencils that
-// lie back to back, or strided ones) or the periodic wrap (strided), of enough rows, with nothing asked for
-// but f' (the assembled rows of compact_fd6 and its halo ends stay with the plan-driven kernels).
+// Whether a launch runs on the constant-coefficient kernels: walls at both ends (unit-stride pencils in
+// planes that lie back to back or apart, or strided ones) or the periodic wrap (strided), of enough rows, with
+// nothing asked for but f' (the assembled rows of compact_fd6 and its halo ends stay with the plan-driven kernels).
 static bool use_uniform(const DerivSpec *sp, int nspec, const AxisGeom &g, bool f64) {
     if (g.n < uniform_min(f64) || g.n > 1024) return false;
     const bool unit = g.srow == 1;
     int M, G, S;
     if (!unit && !seg_shape(g.n, f64, 0, 1, M, G, S)) return false;
-    if (unit && (g.sa != g.n || (g.nb > 1 && g.sb != (long)g.n * g.na))) return false;
+    if (unit && (g.sa != g.n || (g.nb > 1 && g.sb < (long)g.n * g.na))) return false;
     for (int i = 0; i < nspec; i++) {
         const DerivSpec &s = sp[i];
         const bool wall = s.lo_kind == END_WALL && s.hi_kind == END_WALL;

@@ -27,17 +27,23 @@ __global__ __launch_bounds__(256) void k_deriv_line(const DerivLaunch<T> L, cons
     if (id0 >= np) return;
     const unsigned id = id0 + pl;
     const bool active = pl < ppw && id < np;
-    const long at0 = (long)id0 * n, total = (long)np * n - at0;   // values from the wavefront's first pencil on
-    const unsigned at = active ? (unsigned)(pl * n + j * MR) : 0u;   // the lane's first row, from there
+    // values from the wavefront's first pencil on, and the lane's first row from there
+    long at0 = (long)id0 * n, total = (long)np * n - at0, at = active ? (long)(pl * n + j * MR) : 0;
+    unsigned a = id, b = 0;
+    const bool apart = L.nb > 1 && L.sb != (long)L.na * n;   // planes of pencils not back to back
+    if (L.nb > 1 && (apart || J.glo || J.ghi || J.mul_a || J.mul_b)) {
+        b = id / (unsigned)L.na;
+        a = id - b * (unsigned)L.na;
+    }
+    if (apart) {
+        at0 = 0;
+        total = (long)(L.nb - 1) * L.sb + (long)L.na * n;
+        at = active ? (long)a * n + (long)b * L.sb + j * MR : 0;
+    }
     LineShape<MR, REM> G(n, nl, j, active);
     T v[MR], x[MR];
     line_load<T, MR>(J.in + at0, at, total, G, v);
     T lo_val = T(0), hi_val = T(0);
-    unsigned a = id, b = 0;
-    if ((J.glo || J.ghi || J.mul_a || J.mul_b) && L.nb > 1) {
-        b = id / (unsigned)L.na;
-        a = id - b * (unsigned)L.na;
-    }
     if (J.glo || J.ghi) {
         const long gbase = (long)a * J.g_a + (long)b * J.g_b;
         if (G.first && J.glo) lo_val = J.glo[gbase];
@@ -86,7 +92,7 @@ hipError_t launch_deriv_line(const DerivLaunch<T> &L0, int order, hipStream_t st
     DerivLaunch<T> L = L0;
     const int MR = L.M, nl = L.S;
     if ((MR != 8 && MR != 16) || nl != (L.n + MR - 1) / MR || nl > 64 || L.njobs < 1 || L.njobs > kMaxJobs ||
-        L.srow != 1 || L.sa != L.n || (L.nb > 1 && L.sb != (long)L.n * L.na) || (long)L.na * L.nb > 0x7fffff00L)
+        L.srow != 1 || L.sa != L.n || (L.nb > 1 && L.sb < (long)L.n * L.na) || (long)L.na * L.nb > 0x7fffff00L)
         return hipErrorInvalidValue;
     const int ppw = 64 / nl;
     L.M = ppw;

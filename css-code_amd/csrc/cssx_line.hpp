@@ -63,10 +63,11 @@ __device__ __forceinline__ void line_load(const T *__restrict__ p, long at, long
     }
 }
 
-template <typename T, int MR, int REM>
-__device__ __forceinline__ void line_store(T *__restrict__ p, long at, const LineShape<MR, REM> &G, const T (&x)[MR]) {
+// (`at` long, or unsigned from a base that is the same for the wavefront: a 32-bit lane offset in bytes)
+template <typename T, int MR, int REM, class I>
+__device__ __forceinline__ void line_store(T *__restrict__ p, I at, const LineShape<MR, REM> &G, const T (&x)[MR]) {
     if (REM == 0 || !G.last || G.m == MR) {
-        __builtin_memcpy(p + at, x, sizeof(x));
+        __builtin_memcpy((char *)p + at * (I)sizeof(T), x, sizeof(x));
         return;
     }
     // the last lane's m < MR rows in pieces of 8, 4, 2 and 1 (m is wave-uniform; one store per set bit)
@@ -74,7 +75,7 @@ __device__ __forceinline__ void line_store(T *__restrict__ p, long at, const Lin
         constexpr int C = decltype(cnt)::value;
 #pragma unroll
         for (int f = 0; f + C <= MR; f += C)
-            if (f == from) __builtin_memcpy(p + at + f, &x[f], C * sizeof(T));
+            if (f == from) __builtin_memcpy((char *)p + (at + (I)f) * (I)sizeof(T), &x[f], C * sizeof(T));
     };
     int from = 0;
     if constexpr (MR > 8) {
@@ -85,13 +86,77 @@ __device__ __forceinline__ void line_store(T *__restrict__ p, long at, const Lin
     if (G.m & 1) piece(std::integral_constant<int, 1>{}, from);
 }
 
+// Pencils that stay within a wavefront pass nothing to its neighbours
+struct LineWithin {
+    static constexpr bool ON = false;
+};
+// Pencils cut by the end of a wavefront (lanes of a workgroup in one strip): what one side of the cut needs
+// from the other goes through LDS, the six rows next to it for all fields at once and the carry of each
+// recurrence per field, in words that one field and direction owns (one barrier per exchange, none to protect a
+// word's reuse).  A carry dies before the far end of a wavefront, so the sender needs none of its own.
+// The lanes are laid so that the cut is never within the first lanes of a pencil (its lower-wall
+// correction stays in its wavefront) nor before its last lane (rows n-2 and n-1).
+template <typename T, int NF, int NW>
+struct LineCut {
+    T rows[NF][NW][6], up[NF][NW], dn[NF][NW];
+};
+template <typename T, int MR, int NF, int NW>
+struct LineAcross {
+    static constexpr bool ON = true;
+    LineCut<T, NF, NW> &L;
+    int f, w, lane;          // field, wavefront, lane
+    bool from_below, from_above;   // the lane belongs to a pencil cut at its wavefront's lower / upper end
+    T q_below, q_above;      // (-a)^(rows between the cut and the lane)
+    static __device__ __forceinline__ void barrier() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
+    // posts the lane's edge rows of field k (a barrier follows)
+    __device__ __forceinline__ void post(int k, const T (&v)[MR]) {
+        if (lane == 63) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) L.rows[k][w][i] = v[MR - 4 + i];
+        }
+        if (lane == 0) {
+            L.rows[k][w][4] = v[0];
+            L.rows[k][w][5] = v[1];
+        }
+    }
+    __device__ __forceinline__ void window(T (&lo)[4], T (&hi)[2]) const {
+        const int b = w > 0 ? w - 1 : 0, a = w < NW - 1 ? w + 1 : w;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const T t = L.rows[f][b][i];
+            lo[i] = lane == 0 ? t : lo[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const T t = L.rows[f][a][4 + i];
+            hi[i] = lane == 63 ? t : hi[i];
+        }
+    }
+    __device__ __forceinline__ T carry_up(T out) {
+        if (lane == 63) L.up[f][w] = out;
+        barrier();
+        const T t = L.up[f][w > 0 ? w - 1 : 0];
+        return from_below ? q_below * t : T(0);
+    }
+    __device__ __forceinline__ T carry_down(T out) {
+        if (lane == 0) L.dn[f][w] = out;
+        barrier();
+        const T t = L.dn[f][w < NW - 1 ? w + 1 : w];
+        return from_above ? q_above * t : T(0);
+    }
+};
+
 // The derivative of the wavefront's pencils (walls at both ends), times `scale`, in x; row n-1 comes back
 // as the return value of the lane that holds row n-2 (see line_last).  lo_val / hi_val: the prescribed
 // wall derivatives in index units, read on the lanes of rows 0 and n-2.  v's rows past n-1 are
 // overwritten.
-template <typename T, int ORDER, int MR, int REM>
+template <typename T, int ORDER, int MR, int REM, class X = LineWithin>
 __device__ __forceinline__ T line_solve(const LineShape<MR, REM> &G, T (&v)[MR], int bd, T lo_val, T hi_val, T scale,
-                                        T (&x)[MR]) {
+                                        T (&x)[MR], X cut = X()) {
     using U = Uni<ORDER>;
     // carries that reach `reach` rows span this many lanes
     constexpr int NT = (uni_reach<T, ORDER>() + MR - 1) / MR;
@@ -104,11 +169,12 @@ __device__ __forceinline__ T line_solve(const LineShape<MR, REM> &G, T (&v)[MR],
     for (int k = 0; k < 4; k++) lo[k] = from_prev(v[MR - 4 + k]);
     hi[0] = from_next(v[0]);
     hi[1] = from_next(v[1]);
+    if constexpr (X::ON) cut.window(lo, hi);
     auto f = [&](int k) -> T { return k < 0 ? lo[k + 4] : k < MR ? v[k] : hi[k - MR]; };
     // ---- wall rows
     T r0 = T(0), r1 = T(0), q0 = T(0), q1 = T(0);
     {
-        const T e[6] = {v[0], v[1], v[2], v[3], v[4], v[5]};
+        const T e[6] = {f(0), f(1), f(2), f(3), f(4), f(5)};
         wall_rhs<T, ORDER, false>(e, bd, lo_val, false, scale, r0, r1);
     }
 #pragma unroll
@@ -131,6 +197,7 @@ __device__ __forceinline__ T line_solve(const LineShape<MR, REM> &G, T (&v)[MR],
     T Z = T(0);
 #pragma unroll
     for (int i = 0; i < NT; i++) Z = from_prev(up ? y[MR - 1] + Q * Z : T(0));
+    if constexpr (X::ON) Z += cut.carry_up(up ? y[MR - 1] + Q * Z : T(0));
     // (rows 0, 1 of the lower wall stay zero: lane 0 receives no carry)
 #pragma unroll
     for (int k = 0; k < MR && k < uni_reach<T, ORDER>(); k++) y[k] += (T)uni_pow<ORDER>(k + 1) * Z;
@@ -164,6 +231,7 @@ __device__ __forceinline__ T line_solve(const LineShape<MR, REM> &G, T (&v)[MR],
     Z = T(0);
 #pragma unroll
     for (int i = 0; i < NT; i++) Z = from_next(dn ? xf + Q * Z : T(0));
+    if constexpr (X::ON) Z += cut.carry_down(dn ? xf + Q * Z : T(0));
 #pragma unroll
     for (int k = MR - 1; k >= 0 && MR - k <= uni_reach<T, ORDER>(); k--) x[k] += (T)uni_pow<ORDER>(MR - k) * Z;
     // ---- lower wall: rows 0, 1 and the correction of the rows above, passed up the lanes

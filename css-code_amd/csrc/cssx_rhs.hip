@@ -19,6 +19,8 @@
 //   6. two density sweeps + k_rhs_final: the terms of step 4 at every point, the density terms,
 //      top relaxation, u x B (and -etar curl B with its Ohmic heating), xi_cs and the fused RK4
 //      stage; no tendency field is written and re-read in between
+// Without explicit diffusion and for the theta sizes of line_plan, k_rhs_line takes the place of k_rhs_final, of
+// the theta sweeps of steps 3 and 6 and of the theta walls of step 5 (cssx_rhs_line.hpp).
 // Temperature T = rho^(gamma-1) exp(s/Cv)/((gamma-1)Cv) and 1/rho are recomputed where used
 // instead of being stored (rhs_mpi.f90:377-387).
 #include <hip/hip_runtime.h>
@@ -659,8 +661,9 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_walls_density(Consts<T> c, Prof<T> P, WallPtrs W, T *__restrict__ wall,
                                                        const T *__restrict__ st, const T *__restrict__ B,
                                                        const T *__restrict__ D, const T *__restrict__ L,
-                                                       int lbcr_rho, const T *__restrict__ tw) {
-    const long nt = (long)c.nr * c.nphi, nrr = (long)c.nth * c.nphi, N = c.N;
+                                                       int lbcr_rho, const T *__restrict__ tw, int theta) {
+    // theta = 0: the radial walls alone (k_rhs_line closes the theta walls itself)
+    const long nt = theta ? (long)c.nr * c.nphi : 0, nrr = (long)c.nth * c.nphi, N = c.N;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     // the momentum tendency before the density terms, evaluated at the wall points themselves
     T o0[5], o1[5];
@@ -1095,6 +1098,7 @@ __global__ __launch_bounds__(256) void k_cfl_final(const double *__restrict__ re
 }  // namespace cssx
 
 #include "cssx_sld.hpp"
+#include "cssx_rhs_line.hpp"
 
 // =============================================================================================
 // Host orchestration
@@ -1331,6 +1335,49 @@ static bool sld_fork_ok(cssx_mhd *m, hipStream_t stream) {
     return true;
 }
 
+// How k_rhs_line lays the theta pencils of nth rows over a workgroup's lanes
+struct LinePlan {
+    int waves = 0, nl = 0, pencils = 0, off = 0;   // waves = 0: the sweeps and k_rhs_final serve the size
+    bool cut = false;                              // a pencil spans two wavefronts
+};
+template <typename T>
+constexpr int line_run() { return 4; }   // rows per lane (k_rhs_line)
+// The strip of 1, 2 or 4 wavefronts that leaves the fewest lanes idle; pencils cut by a wavefront's end
+// (two barriers per derivative) only for a tenth more lanes in use.  `off` idle lanes in front move a cut out
+// of a pencil's first lanes and its last one (LineAcross).
+// Against the sweeps and k_rhs_final, RHS / RK4 step: FP32 48x96x96 91 -> 78 us / 559 -> 514, 64x1024x128 681 -> 592
+// / 4183 -> 3588, 128x260x128 406 -> 369 / 2456 -> 2177, 100x33x100 96 -> 89 / 592 -> 593; FP64 128x128x128 390 -> 322
+// / 2216 -> 1869, 64x1000x100 1039 -> 1043 / 6006 -> 5745, but with a ragged last lane 90x151x250 648 -> 724
+// / 3628 -> 3854 and 100x50x100 148 -> 172 / 904 -> 1026 (one wavefront per SIMD, spills): those keep the sweeps.
+template <typename T>
+static LinePlan line_plan(const cssx_mhd *m) {
+    LinePlan best;
+    constexpr int MR = line_run<T>(), reach = sizeof(T) == 8 ? 40 : 20, nt = (reach + MR - 1) / MR;
+    // explicit diffusion reads the theta slots elsewhere; shorter pencils are not solved with constant coefficients
+    if (m->p.laplacian || m->p.slaplacian || m->nth < (sizeof(T) == 8 ? 48 : 32)) return best;
+    if (sizeof(T) == 8 && m->nth % MR) return best;
+    const int nl = (m->nth + MR - 1) / MR;
+    double use = 0.0;
+    for (int waves = 1; waves <= 4; waves *= 2)
+        for (int pencils = 64 * waves / nl; pencils > 0; pencils--) {
+            for (int off = 0; off + pencils * nl <= 64 * waves; off++) {
+                bool cut = false, ok = true;
+                for (int w = 1; w < waves; w++) {
+                    const int s = 64 * w - off, j = s % nl;
+                    if (s <= 0 || s >= pencils * nl || j == 0) continue;
+                    cut = true;
+                    ok = ok && j > nt && j < nl - 1;
+                }
+                const double u = (double)(pencils * nl) / (64 * waves) * (cut ? 1.0 : 1.1);
+                if (ok && u > use * 1.001) {
+                    use = u;
+                    best = {waves, nl, pencils, off, cut};
+                }
+            }
+        }
+    return best;
+}
+
 // one batched derivative launch along an axis
 template <typename T>
 static int derivs_axis(cssx_mhd *m, int axis, DerivSpec *specs, int ns, hipStream_t st) {
@@ -1471,6 +1518,35 @@ static int rhs_impl(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
 }
 
 template <typename T>
+static void launch_rhs_line(const LinePlan &lp, bool mag, hipStream_t stream, const Consts<T> &c, const Prof<T> &P, const T *st,
+                            const T *B, const T *dr_rho, T *dv, const StageFuse<T> &F, const float *ext, const T *D,
+                            const LineTheta<T> &H) {
+    constexpr int MR = line_run<T>();
+    const long np = (long)c.nr * c.nphi;
+    const dim3 grid((unsigned)((np + lp.pencils - 1) / lp.pencils)), block(64 * lp.waves);
+    auto run = [&](auto rem, auto mg, auto ct) {
+        hipLaunchKernelGGL((k_rhs_line<T, MR, decltype(rem)::value, decltype(mg)::value, decltype(ct)::value>), grid, block, 0,
+                           stream, c, P, st, B, dr_rho, dv, F, ext, D, H);
+    };
+    auto with_rem = [&](auto mg) {
+        auto cut = [&](auto rem) {
+            if (lp.cut) run(rem, mg, std::true_type{});
+            else run(rem, mg, std::false_type{});
+        };
+        if constexpr (sizeof(T) == 4) {
+            switch (c.nth % MR) {
+            case 1: cut(std::integral_constant<int, 1>{}); return;
+            case 2: cut(std::integral_constant<int, 2>{}); return;
+            case 3: cut(std::integral_constant<int, 3>{}); return;
+            }
+        }
+        cut(std::integral_constant<int, 0>{});
+    };
+    if (mag) with_rem(std::true_type{});
+    else with_rem(std::false_type{});
+}
+
+template <typename T>
 static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream, const StageFuse<T> *F,
                     T *sld_dif, bool fork_closure) {
     int rc = CSSX_OK;
@@ -1526,7 +1602,9 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
     };
     // the theta-wall block for the density wall closure: without explicit diffusion (whose
     // viscous terms the closure would read too)
-    T *tw = (!c.slap && !c.lap) ? S.tw : nullptr;
+    const LinePlan lp = line_plan<T>(m);
+    const bool line = lp.waves > 0;
+    T *tw = (!c.slap && !c.lap && !line) ? S.tw : nullptr;
     const long twM = 2L * m->nr * m->nphi;
     // 3. derivative sweeps
     {
@@ -1548,7 +1626,19 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
                 th[k].tap_side = twM / 2;
             }
         }
-        if ((rc = derivs_axis<T>(m, CSSX_AXIS_THETA, th, mag ? 6 : 4, stream))) return fail(rc);
+        if (line) {
+            // the final kernel solves the theta derivatives; only the density closure of the radial walls
+            // reads them elsewhere, on the two wall planes
+            AxisGeom g;
+            axis_geometry(CSSX_AXIS_THETA, m->nth, m->nphi, m->nr, g);
+            g.nb = 2;
+            g.sb *= m->nr - 1;
+            for (DerivSpec &s : th) s.g_b *= m->nr - 1;
+            if ((rc = run_derivs(th, mag ? 6 : 4, g, sizeof(T) == 8 ? CSSX_PREC_F64 : CSSX_PREC_F32, stream)))
+                return fail(rc);
+        } else if ((rc = derivs_axis<T>(m, CSSX_AXIS_THETA, th, mag ? 6 : 4, stream))) {
+            return fail(rc);
+        }
         DerivSpec ph[7] = {spec<T>(m, CSSX_AXIS_PHI, rho, D + D_PRHO * N, 0, nullptr, nullptr),
                            spec<T>(m, CSSX_AXIS_PHI, v, D + D_PV * N, 0, nullptr, nullptr),
                            spec<T>(m, CSSX_AXIS_PHI, w, D + D_PW * N, 0, nullptr, nullptr),
@@ -1617,18 +1707,18 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
     // 4-5. density wall derivatives from the momentum tendency, which k_walls_density evaluates
     //      (every term before the density terms) at the wall points themselves
     {
-        long nw = std::max((long)m->nr * m->nphi, (long)m->nth * m->nphi);
+        const long nw = line ? (long)m->nth * m->nphi : std::max((long)m->nr * m->nphi, (long)m->nth * m->nphi);
         if (tw)
             hipLaunchKernelGGL(k_walls_gather<T>, dim3(nblocks((long)m->nr * m->nphi, 256)), dim3(256), 0, stream, c,
                                st, (const T *)B, (const T *)D, tw);
         hipLaunchKernelGGL(k_walls_density<T>, dim3(nblocks(nw, 256)), dim3(256), 0, stream, c, P, W, wall, st,
-                           (const T *)B, (const T *)D, (const T *)L, ibcr[1], (const T *)tw);
+                           (const T *)B, (const T *)D, (const T *)L, ibcr[1], (const T *)tw, line ? 0 : 1);
     }
     // 6. density sweeps + every pointwise term, the density terms and the stage in one kernel
     {
         DerivSpec th = spec<T>(m, CSSX_AXIS_THETA, rho, D + D_THRHO * N, ibct[1], wall + W.off_trho_lo,
                                wall + W.off_trho_hi);
-        if ((rc = derivs_axis<T>(m, CSSX_AXIS_THETA, &th, 1, stream))) return fail(rc);
+        if (!line && (rc = derivs_axis<T>(m, CSSX_AXIS_THETA, &th, 1, stream))) return fail(rc);
         DerivSpec rr = spec<T>(m, CSSX_AXIS_R, rho, D + D_RRHO * N, ibcr[1], wall + W.off_rrho_lo,
                                wall + W.off_rrho_hi, nullptr, P.dxdr);
         if ((rc = derivs_axis<T>(m, CSSX_AXIS_R, &rr, 1, stream))) return fail(rc);
@@ -1648,7 +1738,7 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
         // explicit-diffusion fields with Laplacian (SLaplacian); the plain RHS writes 8 (5)
         // tendencies, a fused stage moves the stage traffic of every field instead
         const bool mag = m->p.magnetic;
-        const double reads = (mag ? 29.0 : 20.0) + (c.lap ? 18.0 : c.slap ? 3.0 : 0.0);
+        const double reads = (mag ? 29.0 : 20.0) - (line ? (mag ? 7.0 : 5.0) : 0.0) + (c.lap ? 18.0 : c.slap ? 3.0 : 0.0);
         const double fb = !F ? (mag ? 8.0 : 5.0) * sizeof(T)
                           : sizeof(T) == 8 ? (FF.stage == 1 ? 24.0 + (FF.dif ? 8.0 : 0.0) : FF.stage < 4 ? 32.0 : 24.0) * m->nv
                                            : (FF.stage == 1 ? 12.0 + (FF.dif ? 4.0 : 0.0) : FF.stage < 4 ? 16.0 : 24.0) * m->nv;
@@ -1657,10 +1747,27 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
             (void)hipStreamSynchronize(m->sld_side);
             return CSSX_EHIP;
         }
-        CSSX_TIMED(CSSX_PHASE_RHS_FINAL, stream, reads * N * sizeof(T) + (fb + fo) * N + (ext ? 32.0 * N : 0.0),
-                   hipLaunchKernelGGL(k_rhs_final<T>, dim3(nb), dim3(256), 0, stream, c, P, st, B,
-                                      (const T *)(D + D_THRHO * N), (const T *)(D + D_RRHO * N), dv, FF, ext,
-                                      (const T *)D, (const T *)L));
+        const double bytes = reads * N * sizeof(T) + (fb + fo) * N + (ext ? 32.0 * N : 0.0);
+        if (line) {
+            LineTheta<T> H;
+            H.bw = ibct[2]; H.bv = ibct[3]; H.bu = ibct[4]; H.bs = ibct[5]; H.bbp = ibct[8]; H.bbr = ibct[9]; H.brho = ibct[1];
+            H.tv_lo = wall + W.off_tv_lo; H.tv_hi = wall + W.off_tv_hi;
+            H.tbp_lo = wall + W.off_tbp_lo; H.tbp_hi = wall + W.off_tbp_hi;
+            H.scale = (T)m->grid.dti;
+            H.neu = (T)(1.0 / m->grid.dti);
+            H.nl = lp.nl;
+            H.pencils = lp.pencils;
+            H.off = lp.off;
+            H.inv_nl = (65536u + lp.nl - 1) / lp.nl;
+            CSSX_TIMED(CSSX_PHASE_RHS_FINAL, stream, bytes,
+                       launch_rhs_line<T>(lp, mag, stream, c, P, st, (const T *)B, (const T *)(D + D_RRHO * N), dv, FF, ext,
+                                          (const T *)D, H));
+        } else {
+            CSSX_TIMED(CSSX_PHASE_RHS_FINAL, stream, bytes,
+                       hipLaunchKernelGGL(k_rhs_final<T>, dim3(nb), dim3(256), 0, stream, c, P, st, B,
+                                          (const T *)(D + D_THRHO * N), (const T *)(D + D_RRHO * N), dv, FF, ext,
+                                          (const T *)D, (const T *)L));
+        }
     }
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
