@@ -118,11 +118,11 @@ struct StageRun {
             for (int q = 0; q < MR; q++) y[iv][q] = y[iv][q] + F.dt * (double)s[iv][q];
             bound_run(iv, G, it0, ir, y[iv], F.f, c.nr, F.sr1_64);
             line_store<double, MR>(F.y0 + o, at, G, y[iv]);
-            if constexpr (!F64) {
+            if (!F64 && !F.last) {
                 const double bg = iv == 0 ? F.rbar64[ir] : iv == 4 ? F.sbar64[ir] : 0.0;
 #pragma unroll
-                for (int q = 0; q < MR; q++) s[iv][q] = (float)(y[iv][q] - bg);
-                line_store<float, MR>((float *)F.y0f + o, at, G, s[iv]);
+                for (int q = 0; q < MR; q++) s[iv][q] = (T)(y[iv][q] - bg);
+                line_store<T, MR>(F.y0f + o, at, G, s[iv]);
             }
         }
     }
