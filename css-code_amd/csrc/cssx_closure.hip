@@ -54,6 +54,8 @@ __device__ __forceinline__ float erf_as(float x) {
     return __builtin_copysignf(1.0f - poly * exp_neg_sq(ax), x);
 }
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erf_as(z * 0.70710678118654752f)); }
+// 2 gelu(z), for inference: the weights that its results meet are packed halved, which changes no product
+__device__ __forceinline__ float gelu2(float z) { return z * (1.0f + erf_as(z * 0.70710678118654752f)); }
 __device__ __forceinline__ float gelu_grad(float z) {
     return 0.5f * (1.0f + erf_as(z * 0.70710678118654752f)) + z * 0.39894228040143268f * exp_neg_sq(0.70710678118654752f * z);
 }
@@ -374,11 +376,11 @@ __global__ __launch_bounds__(256) void k_pack_infer(const float *__restrict__ W,
     } else if (i < (long)kH * kS1 + (long)kH * kS2) {
         const long j = i - (long)kH * kS1;
         const int o = (int)(j / kS2), k = (int)(j % kS2);
-        pk[i] = k < kH ? (cssx_bf16)W[oW2 + (long)perm_unit(k >> 5, k & 31) * kH + o] : zero;
+        pk[i] = k < kH ? (cssx_bf16)(0.5f * W[oW2 + (long)perm_unit(k >> 5, k & 31) * kH + o]) : zero;   // (gelu2)
     } else if (i < kPackBf) {
         const long j = i - (long)kH * kS1 - (long)kH * kS2;
         const int o = (int)(j / kS2), k = (int)(j % kS2);
-        pk[i] = (k < kH && o < kOut) ? (cssx_bf16)W[oW3 + (long)perm_unit(k >> 5, k & 31) * kOut + o] : zero;
+        pk[i] = (k < kH && o < kOut) ? (cssx_bf16)(0.5f * W[oW3 + (long)perm_unit(k >> 5, k & 31) * kOut + o]) : zero;
     } else if (i < kPackBf + kPackF) {
         const int j = (int)(i - kPackBf);
         float *bf = reinterpret_cast<float *>(pk + kPackBf);
@@ -451,7 +453,7 @@ __global__ __launch_bounds__(512) void k_closure_infer(const T *__restrict__ st,
 #pragma unroll
         for (int nb = 0; nb < 8; nb++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) h[nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu(acc[nb][r] + b1[nb * 16 + 4 * g + r]);
+            for (int r = 0; r < 4; r++) h[nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu2(acc[nb][r] + b1[nb * 16 + 4 * g + r]);
         // layer 2
 #pragma unroll
         for (int nb = 0; nb < 8; nb++) acc[nb] = cssx_f32x4{0.f, 0.f, 0.f, 0.f};
@@ -465,7 +467,7 @@ __global__ __launch_bounds__(512) void k_closure_infer(const T *__restrict__ st,
 #pragma unroll
         for (int nb = 0; nb < 8; nb++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) h[nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu(acc[nb][r] + b2[nb * 16 + 4 * g + r]);
+            for (int r = 0; r < 4; r++) h[nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu2(acc[nb][r] + b2[nb * 16 + 4 * g + r]);
         // layer 3 (8 outputs padded to one 16-row block)
         cssx_f32x4 y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -490,6 +492,13 @@ __global__ __launch_bounds__(512) void k_closure_infer(const T *__restrict__ st,
 // instead of one per K step), converts them to FP32 (background subtracted as above) into its
 // slot of LDS, and the K steps gather their B operands from there; the standardization tables
 // sit in LDS beside the packed weights.
+//
+// Bound by the vector ALU (two GELUs of 128 activations per point) and by LDS reads, which the layout keeps low:
+// a wavefront takes two tiles at a time, so that every weight fragment it reads serves two matrix
+// products (their B operands stay in registers, 28 per tile), and a footprint point's eight
+// fields lie in two 16-byte quarters, as the tables' do, instead of 24 four-byte reads per K step.
+// 64x128x256 FP32: one tile at a time 540 us, two 437, with gelu2 423 (448 TFLOP/s; the vector ALU's share
+// alone is 375); the next pair's footprints asked for before the products: 436.
 constexpr int kFoot = 8 * 3 * 3 * 18;   // footprint values per tile
 constexpr int kInferWaves = 8;
 constexpr size_t kInferRowsBytes = kPackBytes + 2 * kFeat * sizeof(float) + (size_t)kInferWaves * kFoot * sizeof(float);
@@ -511,106 +520,161 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
         const uint4 *src = reinterpret_cast<const uint4 *>(pk);
         for (int i = threadIdx.x; i < (int)(kPackBytes / 16); i += blockDim.x) lds4[i] = src[i];
     }
-    float *xm = reinterpret_cast<float *>(reinterpret_cast<unsigned char *>(lds4) + kPackBytes);
-    float *xs = xm + kFeat;
-    for (int i = threadIdx.x; i < kFeat; i += blockDim.x) {
-        xm[i] = xmean[i];
-        xs[i] = xistd[i];
+    // standardization by neighbour: table q of neighbour nbh holds fields 4q .. 4q+3
+    float4 *xm = reinterpret_cast<float4 *>(reinterpret_cast<unsigned char *>(lds4) + kPackBytes);
+    float4 *xs = xm + 2 * 27;
+    for (int i = threadIdx.x; i < kFeat; i += blockDim.x) {   // i = e * 27 + nbh
+        const int e = i / 27, at = ((e >> 2) * 27 + (i - 27 * e)) * 4 + (e & 3);
+        reinterpret_cast<float *>(xm)[at] = xmean[i];
+        reinterpret_cast<float *>(xs)[at] = xistd[i];
     }
     __syncthreads();
     const cssx_bf16 *W1T = reinterpret_cast<const cssx_bf16 *>(lds4);
     const cssx_bf16 *W2P = W1T + kH * kS1, *W3P = W2P + kH * kS2;
     const float *b1 = reinterpret_cast<const float *>(W1T + kPackBf), *b2 = b1 + kH, *b3 = b2 + kH;
-    const int lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15, wv = threadIdx.x >> 6;
-    float *fp = xs + kFeat + wv * kFoot;
+    const int lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    float4 *fp = xs + 2 * 27 + wv * (kFoot / 4);
     // footprint slot of the lane; lanes >= 54 are idle (their loads stay in bounds, unused)
     const int dp = min(lane / 18, 2), tt = lane - 18 * (lane / 18);
     const __amdgpu_buffer_rsrc_t rs = field_rsrc(st);
-    const long ntiles = N / 16;
+    const long ntiles = N / 16;   // a field is below 4 GiB / 8 (field_rsrc offsets): tiles count in 32 bits
+    const int ntt = nth / 16;
     const cssx_bf16 zero = (cssx_bf16)0.0f;
-    for (long t = (long)blockIdx.x * kInferWaves + wv; t < ntiles; t += (long)gridDim.x * kInferWaves) {
-        const long p0 = t * 16;
-        const int it0 = (int)(p0 % nth);
-        const long rest = p0 / nth;
-        const int ip = (int)(rest % nphi), ir = (int)(rest / nphi);
-        // footprint: value f = ((e*3 + dr)*3 + dp)*18 + tt of field e at r row ir+dr-1 (clamped),
-        // phi ip+dp-1 (periodic), theta it0+tt-1 (clamped).  Lane l < 54 owns dp = l/18 and
-        // tt = l%18, and pass k = 3e + dr fills slot 54k + l: the lane's offset is fixed per tile
-        // and each pass adds a uniform (scalar) offset, so a load costs no address arithmetic.
+    // tile t's footprint: value (e, dr, dp, tt) of field e at r row ir+dr-1 (clamped), phi ip+dp-1
+    // (periodic), theta it0+tt-1 (clamped).  Lane l < 54 owns dp = l/18 and tt = l%18, and k = 3e + dr is a
+    // pass: the lane's offset is fixed per tile and each pass adds a uniform (scalar) offset, so a load
+    // costs no address arithmetic.
+    auto fetch = [&](long t, T(&v)[24]) __attribute__((always_inline)) {
+        const unsigned q0 = (unsigned)t / (unsigned)ntt, ir = q0 / (unsigned)nphi;
+        const int it0 = (int)((unsigned)t - q0 * ntt) * 16, ip = (int)(q0 - ir * nphi);
         const int jt = min(max(it0 + tt - 1, 0), nth - 1);
         int jp = ip + dp - 1;
         jp = jp < 0 ? jp + nphi : (jp >= nphi ? jp - nphi : jp);
         const unsigned voff = (unsigned)(((long)jp * nth + jt) * (long)sizeof(T));
-        float v[24];
 #pragma unroll
         for (int k = 0; k < 24; k++) {
-            const int e = k / 3, dr = k % 3;
-            const int jr = min(max(ir + dr - 1, 0), nr - 1);
-            const T raw = bload<T>(rs, voff, (unsigned)(((long)e * N + (long)jr * nphi * nth) * (long)sizeof(T)));
-            if (!fluct && e == 0) v[k] = (float)((double)raw - (double)rbar[jr]);
-            else if (!fluct && e == 4) v[k] = (float)((double)raw - (double)sbar[jr]);
-            else v[k] = (float)raw;
+            const int e = k / 3, jr = min(max((int)ir + k % 3 - 1, 0), nr - 1);
+            v[k] = bload<T>(rs, voff, (unsigned)(((long)e * N + (long)jr * nphi * nth) * (long)sizeof(T)));
+        }
+    };
+    // the tile's B operands of layer 1
+    using Words = int __attribute__((ext_vector_type(4)));
+    auto features = [&](long t, const T(&v)[24], cssx_bf16x8(&b)[kKp1 / 32]) __attribute__((always_inline)) {
+        const int ir = (int)((unsigned)t / (unsigned)ntt / (unsigned)nphi);
+        float x[24];
+#pragma unroll
+        for (int k = 0; k < 24; k++) {
+            const int e = k / 3, jr = min(max(ir + k % 3 - 1, 0), nr - 1);
+            if (!fluct && e == 0) x[k] = (float)((double)v[k] - (double)rbar[jr]);
+            else if (!fluct && e == 4) x[k] = (float)((double)v[k] - (double)sbar[jr]);
+            else x[k] = (float)v[k];
         }
         wave_sync();   // the previous tile's reads of fp are done
         if (lane < 54) {
 #pragma unroll
-            for (int k = 0; k < 24; k++) fp[54 * k + lane] = v[k];
+            for (int dr = 0; dr < 3; dr++)
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+                    fp[162 * q + 54 * dr + lane] = make_float4(x[12 * q + dr], x[12 * q + 3 + dr], x[12 * q + 6 + dr], x[12 * q + 9 + dr]);
         }
         wave_sync();
-        cssx_f32x4 acc[8];
-#pragma unroll
-        for (int nb = 0; nb < 8; nb++) acc[nb] = cssx_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < kKp1 / 32; ks++) {
-            cssx_bf16x8 b;
-            const int nbh = 4 * ks + g;   // this lane's neighbour; its 8 slots are the 8 fields
-            if (nbh < 27) {
-                const int dr = nbh / 9, dp = (nbh / 3) % 3, dt = nbh % 3;
-                const float *f0 = fp + (dr * 3 + dp) * 18 + li + dt;
+            const int nbh = min(4 * ks + g, 26);   // this lane's neighbour; its 8 slots are the 8 fields
+            const int dr = nbh / 9, dq = (nbh / 3) % 3, dt = nbh % 3;
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int q = e * 27 + nbh;
-                    b[e] = (cssx_bf16)((f0[e * 162] - xm[q]) * xs[q]);
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) b[e] = zero;
+            for (int q = 0; q < 2; q++) {
+                const float4 f = fp[162 * q + (dr * 3 + dq) * 18 + li + dt], m = xm[27 * q + nbh], d = xs[27 * q + nbh];
+                b[ks][4 * q] = (cssx_bf16)((f.x - m.x) * d.x);
+                b[ks][4 * q + 1] = (cssx_bf16)((f.y - m.y) * d.y);
+                b[ks][4 * q + 2] = (cssx_bf16)((f.z - m.z) * d.z);
+                b[ks][4 * q + 3] = (cssx_bf16)((f.w - m.w) * d.w);
             }
+            if (4 * ks + 3 > 26 && 4 * ks + g > 26) {   // the padding of K
+#pragma unroll
+                for (int e = 0; e < 8; e++) b[ks][e] = zero;
+            }
+            // the operand is complete here: left to its use, the arithmetic would sink there and keep its 24 inputs
+            // in registers instead of its 4 results
+            Words w = __builtin_bit_cast(Words, b[ks]);
+            asm volatile("" : "+v"(w));
+            b[ks] = __builtin_bit_cast(cssx_bf16x8, w);
+        }
+    };
+    const long step = 2L * gridDim.x * kInferWaves;
+    long t = 2 * ((long)blockIdx.x * kInferWaves + wv);
+    for (; t < ntiles; t += step) {
+        const bool two = t + 1 < ntiles;   // else the second half repeats the last tile and stores nothing
+        // one lane address per array, taken anew for each pair (constant offsets from there): kept across the loop
+        // the addresses and the values behind them would not fit the registers
+        int fresh = 0;
+        asm volatile("" : "+s"(fresh));
+        const cssx_bf16 *w1 = W1T + (li * kS1 + 8 * g + fresh), *w2 = W2P + (li * kS2 + 8 * g + fresh);
+        const cssx_bf16 *w3 = W3P + (li * kS2 + 8 * g + fresh);
+        cssx_bf16x8 b[2][kKp1 / 32];
+        T raw[2][24];
+        fetch(t, raw[0]);
+        fetch(two ? t + 1 : t, raw[1]);
+        features(t, raw[0], b[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        features(two ? t + 1 : t, raw[1], b[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        cssx_f32x4 acc[2][8];
+        cssx_bf16x8 h[2][4];
+        auto clear = [&]() {
+#pragma unroll
+            for (int nb = 0; nb < 8; nb++) acc[0][nb] = acc[1][nb] = cssx_f32x4{0.f, 0.f, 0.f, 0.f};
+        };
+        auto activate = [&](const float *bias) __attribute__((always_inline)) {
 #pragma unroll
             for (int nb = 0; nb < 8; nb++) {
-                const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(W1T + (nb * 16 + li) * kS1 + ks * 32 + 8 * g);
-                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nb], 0, 0, 0);
+                const float4 bb = *reinterpret_cast<const float4 *>(bias + nb * 16);
+                const float bv[4] = {bb.x, bb.y, bb.z, bb.w};
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) h[u][nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu2(acc[u][nb][r] + bv[r]);
             }
-        }
-        cssx_bf16x8 h[4];
+        };
+        clear();
 #pragma unroll
-        for (int nb = 0; nb < 8; nb++)
+        for (int ks = 0; ks < kKp1 / 32; ks++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) h[nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu(acc[nb][r] + b1[nb * 16 + 4 * g + r]);
+            for (int nb = 0; nb < 8; nb++) {
+                const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(w1 + nb * 16 * kS1 + ks * 32);
 #pragma unroll
-        for (int nb = 0; nb < 8; nb++) acc[nb] = cssx_f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int u = 0; u < 2; u++) acc[u][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[u][ks], acc[u][nb], 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        activate(b1 + (4 * g + fresh));
+        __builtin_amdgcn_sched_barrier(0);
+        clear();
 #pragma unroll
         for (int ks = 0; ks < 4; ks++)
 #pragma unroll
             for (int nb = 0; nb < 8; nb++) {
-                const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(W2P + (nb * 16 + li) * kS2 + ks * 32 + 8 * g);
-                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[ks], acc[nb], 0, 0, 0);
+                const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(w2 + nb * 16 * kS2 + ks * 32);
+#pragma unroll
+                for (int u = 0; u < 2; u++) acc[u][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[u][ks], acc[u][nb], 0, 0, 0);
             }
-#pragma unroll
-        for (int nb = 0; nb < 8; nb++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) h[nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu(acc[nb][r] + b2[nb * 16 + 4 * g + r]);
-        cssx_f32x4 y = {0.f, 0.f, 0.f, 0.f};
+        __builtin_amdgcn_sched_barrier(0);
+        activate(b2 + (4 * g + fresh));
+        __builtin_amdgcn_sched_barrier(0);
+        cssx_f32x4 y[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
-            const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(W3P + li * kS2 + ks * 32 + 8 * g);
-            y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[ks], y, 0, 0, 0);
+            const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(w3 + ks * 32);
+#pragma unroll
+            for (int u = 0; u < 2; u++) y[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[u][ks], y[u], 0, 0, 0);
         }
         if (g < 2) {
+            const int o = 4 * g + fresh;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int o = 4 * g + r;
-                ext[(long)o * N + p0 + li] = (y[r] + b3[o]) * ystd[o] + ymean[o];
+                float *e = ext + ((long)(o + r) * N + t * 16 + li);
+                const float sc = ystd[o + r], of = ymean[o + r], bo = b3[o + r];
+                e[0] = (y[0][r] + bo) * sc + of;
+                if (two) e[16] = (y[1][r] + bo) * sc + of;
             }
         }
     }
@@ -816,7 +880,7 @@ int closure_tendency(cssx_mlp *n, int prec, const void *st, int fluct, const voi
             const void *fr = prec == CSSX_PREC_F64 ? (const void *)k_closure_infer_rows<double>
                                                    : (const void *)k_closure_infer_rows<float>;
             if (int rc = fused_setup(fr, kInferRowsBytes, &ncu)) return rc;
-            const unsigned grid = (unsigned)std::min<long>((long)ncu, (tiles + kInferWaves - 1) / kInferWaves);
+            const unsigned grid = (unsigned)std::min<long>((long)ncu, (tiles + 2 * kInferWaves - 1) / (2 * kInferWaves));
             if (prec == CSSX_PREC_F64)
                 hipLaunchKernelGGL(k_closure_infer_rows<double>, dim3(grid), dim3(64 * kInferWaves), kInferRowsBytes, s,
                                    (const double *)st, N, nr, nphi, nth, fluct, (const double *)rbar,
