@@ -13,10 +13,7 @@ import torch
 
 from . import _lib
 from .model import Config, Model
-
-
-def _stream():
-    return ctypes.c_void_p(int(torch.cuda.current_stream().cuda_stream))
+from .operators import _stream
 
 
 class Solver:
