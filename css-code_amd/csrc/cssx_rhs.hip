@@ -210,23 +210,28 @@ struct Thermo {
     T rho, t;
     T a, b;   // fluctuation form: T/rho = (T_bar/rho_bar)(1+a), T = T_bar (1+b)
 };
-template <typename T>
-__device__ __forceinline__ Thermo<T> thermo(T rho_st, T s_st, int ir, const Consts<T> &c, const Prof<T> &P) {
+template <typename T, bool FL>
+__device__ __forceinline__ Thermo<T> thermo_at(T rho_st, T s_st, T rb, T tbar, const Consts<T> &c) {
     Thermo<T> o;
-    if (c.fluct) {
-        const T rb = P.rbar[ir];
+    if (FL) {
         o.rho = rb + rho_st;
         // log1p/expm1 keep the relative precision of the small departures a, b themselves
         const T lq = log1p(rho_st / rb), e1 = s_st * c.invCv;
         o.b = expm1(c.gamm1 * lq + e1);
         o.a = expm1((c.gamm1 - T(1)) * lq + e1);
-        o.t = P.tbar[ir] * (T(1) + o.b);
+        o.t = tbar * (T(1) + o.b);
     } else {
         o.rho = rho_st;
         o.t = temperature(rho_st, s_st, c);
         o.a = o.b = T(0);
     }
     return o;
+}
+
+template <typename T>
+__device__ __forceinline__ Thermo<T> thermo(T rho_st, T s_st, int ir, const Consts<T> &c, const Prof<T> &P) {
+    return c.fluct ? thermo_at<T, true>(rho_st, s_st, P.rbar[ir], P.tbar[ir], c)
+                   : thermo_at<T, false>(rho_st, s_st, T(0), T(0), c);
 }
 
 template <typename T>
@@ -1396,7 +1401,8 @@ static LinePlan line_plan(const cssx_mhd *m) {
                     cut = true;
                     ok = ok && j > nt && j < nl - 1;
                 }
-                const double u = (double)(pencils * nl) / (64 * waves) * (cut ? 1.0 : 1.1);
+                const int wgs = (m->nphi + pencils - 1) / pencils;   // of one radius
+                const double u = (double)m->nphi * nl / (64.0 * waves * wgs) * (cut ? 1.0 : 1.1);
                 if (ok && u > use * 1.001) {
                     use = u;
                     best = {waves, nl, pencils, off, cut};
@@ -1550,8 +1556,7 @@ static void launch_rhs_line(const LinePlan &lp, bool mag, hipStream_t stream, co
                             const T *B, const T *dr_rho, T *dv, const StageFuse<T> &F, const float *ext, const T *D,
                             const LineTheta<T> &H) {
     constexpr int MR = line_run<T>();
-    const long np = (long)c.nr * c.nphi;
-    const dim3 grid((unsigned)((np + lp.pencils - 1) / lp.pencils)), block(64 * lp.waves);
+    const dim3 grid((unsigned)((c.nphi + lp.pencils - 1) / lp.pencils), (unsigned)c.nr), block(64 * lp.waves);
     auto run = [&](auto rem, auto mg, auto ct) {
         hipLaunchKernelGGL((k_rhs_line<T, MR, decltype(rem)::value, decltype(mg)::value, decltype(ct)::value>), grid, block, 0,
                            stream, c, P, st, B, dr_rho, dv, F, ext, D, H);

@@ -136,12 +136,15 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
     const int n = c.nth, nl = H.nl;
     const int lane = threadIdx.x & 63, s0 = (int)threadIdx.x - H.off;
     const int pl = s0 < 0 ? H.pencils : (int)((unsigned)s0 * H.inv_nl >> 16);
-    const unsigned np = (unsigned)c.nr * (unsigned)c.nphi, id0 = blockIdx.x * (unsigned)H.pencils;
-    const bool active = pl < H.pencils && id0 + pl < np;
+    constexpr bool FL = sizeof(T) == 4;   // fluctuation form (Consts::fluct)
+    const unsigned ip0 = blockIdx.x * (unsigned)H.pencils;
+    const int ir = (int)blockIdx.y;
+    const unsigned id0 = (unsigned)ir * (unsigned)c.nphi + ip0;
+    const bool active = pl < H.pencils && ip0 + pl < (unsigned)c.nphi;
     // lanes without a pencil work along on the first one and store nothing
     const unsigned id = active ? id0 + pl : id0;
     const int j = active ? s0 - pl * nl : 0;
-    const int ir = (int)(id / (unsigned)c.nphi), it0 = j * MR;
+    const int it0 = j * MR;
     const long N = c.N, base = (long)id0 * n;   // the workgroup's first point
     const unsigned at = active ? (unsigned)(pl * n + it0) : 0u;
     const LineShape<MR, REM> G(n, nl, j, active);
@@ -182,8 +185,21 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
         }
         line_last<T, MR>(G, xn1, x);
     };
-    const T ri = P.rinv[ir], rv = P.r[ir], epsr = P.eps[ir];
+    // A workgroup stays within one radius, whose profiles are scalars, and everything small is asked for here: loads
+    // return in order, so one in the middle of the terms waits for whatever is in flight before it.  RK4 step,
+    // against workgroups across radii that read the profiles where they use them: 256x512x1024 FP32 52.6 -> 50.3 ms,
+    // 128x256x512 FP64 12.3 -> 11.9, 90x151x250 FP32 (two steps) 3.85 -> 3.61, 48x96x96 FP32 RHS 77.2 -> 74.0 us.
+    const T ri = P.rinv[ir], rv = P.r[ir], epsr = P.eps[ir], g0 = FL ? P.hres[ir] : -P.grav[ir];
+    const T rb = FL ? P.rbar[ir] : T(0), tbar = FL ? P.tbar[ir] : T(0), dsb = FL ? P.dsbar[ir] : T(0);
+    const T tr = FL ? P.tr[ir] : T(0), drb = FL ? P.drbar[ir] : T(0);
     const T omsq = rv * c.omega0 * c.omega0, om2 = c.om2;
+    T cot[MR], sn[MR], cs[MR], csc[MR];
+    theta(P.cot, cot);
+    theta(P.sn, sn);
+    theta(P.cs, cs);
+    theta(P.csc, csc);
+    const T vl = (G.first && H.tv_lo) ? H.tv_lo[id] : T(0), vh = (G.at_n2 && H.tv_hi) ? H.tv_hi[id] : T(0);
+    const T bl = (MAG && G.first && H.tbp_lo) ? H.tbp_lo[id] : T(0), bh = (MAG && G.at_n2 && H.tbp_hi) ? H.tbp_hi[id] : T(0);
     T W[MR], V[MR], U[MR], rs[MR], Bt[MR], Bp[MR], Br[MR], S[MR];
     field(st, rs);
     field(st + 4 * N, S);
@@ -209,20 +225,15 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
     }
     T Rho[MR], t[MR], ta[MR], tb[MR];
     CSSX_K {
-        const Thermo<T> th = thermo(rs[k], S[k], ir, c, P);
+        const Thermo<T> th = thermo_at<T, FL>(rs[k], S[k], rb, tbar, c);
         Rho[k] = th.rho;
         t[k] = th.t;
         ta[k] = th.a;
         tb[k] = th.b;
     }
-    T xdw[MR], xdv[MR], xdu[MR], xdrho[MR], xds[MR], x[MR], cot[MR];
-    theta(P.cot, cot);
+    T xdw[MR], xdv[MR], xdu[MR], xdrho[MR], xds[MR], x[MR];
     // ---- Source_Theta_Terms (rhs_mpi.f90:812-1027)
     {
-        T sn[MR], cs[MR];
-        theta(P.sn, sn);
-        theta(P.cs, cs);
-        const T g0 = c.fluct ? P.hres[ir] : -P.grav[ir];
         dth(0, W, H.bw, T(0), T(0), x);
         CSSX_K {
             xdw[k] = omsq * sn[k] * cs[k];
@@ -237,7 +248,6 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
             xdv[k] = xdv[k] - ri * V[k] * W[k] * cot[k];
             xdu[k] = xdu[k] + V[k] * (ri * V[k] + om2 * sn[k]);
         }
-        const T vl = (G.first && H.tv_lo) ? H.tv_lo[id] : T(0), vh = (G.at_n2 && H.tv_hi) ? H.tv_hi[id] : T(0);
         dth(1, V, H.bv, vl, vh, x);
         CSSX_K {
             xdv[k] = xdv[k] - W[k] * (x[k] * ri);
@@ -256,7 +266,6 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
         xds[k] = xds[k] - W[k] * wk;
     }
     if constexpr (MAG) {
-        const T bl = (G.first && H.tbp_lo) ? H.tbp_lo[id] : T(0), bh = (G.at_n2 && H.tbp_hi) ? H.tbp_hi[id] : T(0);
         dth(4, Bp, H.bbp, bl, bh, x);
         CSSX_K {
             const T oorho = (T(1) / Rho[k]) * T(kOneOver4Pi) * ri;
@@ -280,8 +289,7 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
     // ---- Phi_Terms (rhs_mpi.f90:1064-1260)
     {
         T oors[MR];
-        theta(P.csc, oors);
-        CSSX_K oors[k] = ri * oors[k];
+        CSSX_K oors[k] = ri * csc[k];
         slot(D_PRHO, x);
         CSSX_K {
             const T wk = x[k] * oors[k];
@@ -330,8 +338,7 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
         xdrho[k] = xdrho[k] - Rho[k] * x[k];
     }
     slot(D_RS, x);
-    if (c.fluct) {
-        const T tbar = P.tbar[ir], dsb = P.dsbar[ir];
+    if constexpr (FL) {
         CSSX_K {
             xdu[k] = xdu[k] - c.gamm1 * (t[k] * x[k] + tbar * tb[k] * dsb);
             xds[k] = xds[k] - U[k] * (x[k] + dsb);
@@ -356,6 +363,8 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
             xdu[k] = xdu[k] - Bp[k] * wk;
         }
     }
+    T drr[MR];
+    field(dr_rho, drr);
     // ---- Density_Terms_Theta: the wall derivatives that zero the normal momentum tendency
     //      (rhs_mpi.f90:1553-1564), from the end points' own lanes
     {
@@ -378,23 +387,21 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
         }
     }
     // ---- Density_Terms_Radial
-    field(dr_rho, x);
-    if (c.fluct) {
-        const T tr = P.tr[ir], drb = P.drbar[ir];
+    if constexpr (FL) {
         CSSX_K {
-            xdu[k] = xdu[k] - c.pconst * ((t[k] * (T(1) / Rho[k])) * x[k] + tr * ta[k] * drb);
-            xdrho[k] = xdrho[k] - U[k] * (x[k] + drb);
+            xdu[k] = xdu[k] - c.pconst * ((t[k] * (T(1) / Rho[k])) * drr[k] + tr * ta[k] * drb);
+            xdrho[k] = xdrho[k] - U[k] * (drr[k] + drb);
         }
     } else {
         CSSX_K {
-            xdrho[k] = xdrho[k] - U[k] * x[k];
-            xdu[k] = xdu[k] - c.pconst * t[k] * (x[k] * (T(1) / Rho[k]));
+            xdrho[k] = xdrho[k] - U[k] * drr[k];
+            xdu[k] = xdu[k] - c.pconst * t[k] * (drr[k] * (T(1) / Rho[k]));
         }
     }
     if (c.top_relax && ir == c.nr - 1) {
-        const T dt_ = c.damp * (c.gamma - T(2)), tbar = P.tbar[ir];
+        const T dt_ = c.damp * (c.gamma - T(2));
         CSSX_K {
-            const T dT = c.fluct ? c.dT0top - tbar * tb[k] : c.T0 - t[k];
+            const T dT = FL ? c.dT0top - tbar * tb[k] : c.T0 - t[k];
             xdrho[k] = xdrho[k] + Rho[k] * dT / (dt_ * t[k]);
             xds[k] = xds[k] - c.Cv * dT / (dt_ * t[k]);
         }
@@ -505,7 +512,7 @@ __global__ __launch_bounds__(256, (MR * sizeof(T) > 16 ? 1 : 2)) void k_rhs_line
                                                      LineTheta<T> H) {
     __shared__ LineCut<T, 7, 4> cut;
     // the last workgroup's last lane may reach past the fields' end
-    if (REM != 0 && blockIdx.x == gridDim.x - 1)
+    if (REM != 0 && blockIdx.x == gridDim.x - 1 && blockIdx.y == gridDim.y - 1)
         rhs_line<T, MR, REM, MAG, CUT, true>(c, P, st, B, dr_rho, dv, F, ext, D, H, cut);
     else
         rhs_line<T, MR, REM, MAG, CUT, false>(c, P, st, B, dr_rho, dv, F, ext, D, H, cut);
