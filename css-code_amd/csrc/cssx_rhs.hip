@@ -67,6 +67,9 @@ struct Prof {
     // momentum residual -g - pconst (T_bar/rho_bar) drbar - (gamma-1) T_bar dsbar (zero on
     // Neumann density walls, truncation-small inside), tr = T_bar/rho_bar
     T *hres = nullptr, *tr = nullptr;
+    // d rho/dr (physical, nr) of a unit wall derivative of the density, in x-space, at the lower and the upper
+    // radial wall; zero where that wall's closure prescribes none
+    T *erl = nullptr, *erh = nullptr;
     // SLD face geometry (diffusion.f90:805-838, 1219-1250, 1316-1348): r face radii rfc (nr+1,
     // 0 on the walls so their flux vanishes), 3/(r_h^3-r_l^3) rv (nr), sin of the theta faces
     // sph (nth+1, 0 on the walls), 1.5(r_h^2-r_l^2)/(r_h^3-r_l^3) rfac (nr),
@@ -334,23 +337,33 @@ inline WallPtrs wall_layout(int nr, int nth, int nphi) {
     return w;
 }
 
+// With B it first applies the Compute_B wall conditions (k_curl_walls) to its wall points: the theta-wall values read B
+// at their own thread's points only, and where a radial wall's thread zeroes one of those they take zero.
 template <typename T>
 __global__ __launch_bounds__(256) void k_walls_state(Consts<T> c, Prof<T> P, WallPtrs W, T *__restrict__ wall,
-                                                     const T *__restrict__ st, const T *__restrict__ B,
+                                                     const T *__restrict__ st, T *__restrict__ B,
                                                      int bot_sf, int top_sf, int bot_flux, int top_flux,
-                                                     int theta_normal) {
-    const long nt = (long)c.nr * c.nphi, nrr = (long)c.nth * c.nphi;
+                                                     int theta_normal, int perf_cond, int bot_radial, int top_radial) {
+    const long nt = (long)c.nr * c.nphi, nrr = (long)c.nth * c.nphi, N = c.N;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const T *w = st + c.N, *v = st + 2 * c.N;
+    const T *w = st + N, *v = st + 2 * N;
     if (i < nt) {   // theta walls (rhs_mpi.f90:410-455): pencil (ip, ir)
-        const int ip = (int)(i % c.nphi), ir = (int)(i / c.nphi);
-        const long q0 = ((long)ir * c.nphi + ip) * c.nth, q1 = q0 + c.nth - 1;
-        wall[W.off_tv_lo + i] = P.cs[0] / P.sn[0] * v[q0];
-        wall[W.off_tv_hi + i] = P.cs[c.nth - 1] / P.sn[c.nth - 1] * v[q1];
+        const int ir = (int)(i / c.nphi);
+        const bool radial = (bot_radial && ir == 0) || (top_radial && ir == c.nr - 1);
+        const long q0 = i * c.nth, q1 = q0 + c.nth - 1;
+        const bool bp_on = c.magnetic && theta_normal && perf_cond && !radial;
+        const T v0 = v[q0], v1 = v[q1], p0 = bp_on ? B[N + q0] : T(0), p1 = bp_on ? B[N + q1] : T(0);
+        wall[W.off_tv_lo + i] = P.cs[0] / P.sn[0] * v0;
+        wall[W.off_tv_hi + i] = P.cs[c.nth - 1] / P.sn[c.nth - 1] * v1;
         if (c.magnetic) {
-            const T *bp = B + c.N;
-            wall[W.off_tbp_lo + i] = theta_normal ? -P.cs[0] / P.sn[0] * bp[q0] : T(0);
-            wall[W.off_tbp_hi + i] = theta_normal ? -P.cs[c.nth - 1] / P.sn[c.nth - 1] * bp[q1] : T(0);
+            wall[W.off_tbp_lo + i] = theta_normal ? -P.cs[0] / P.sn[0] * p0 : T(0);
+            wall[W.off_tbp_hi + i] = theta_normal ? -P.cs[c.nth - 1] / P.sn[c.nth - 1] * p1 : T(0);
+            if (perf_cond) {
+                B[q0] = B[q1] = T(0);
+            } else {
+                B[N + q0] = B[N + q1] = T(0);
+                B[2 * N + q0] = B[2 * N + q1] = T(0);
+            }
         }
     }
     if (i < nrr) {  // radial walls (rhs_mpi.f90:578-637): pencil (it, ip)
@@ -363,6 +376,8 @@ __global__ __launch_bounds__(256) void k_walls_state(Consts<T> c, Prof<T> P, Wal
         wall[W.off_rv_hi + i] = top_sf ? v[q1] / r2 / x2 : v[q1];
         wall[W.off_rs_lo + i] = bot_flux ? (c.slap ? c.s_lap_lo : P.dsdr1[it] / x1) : T(0);
         wall[W.off_rs_hi + i] = top_flux ? (c.slap ? c.s_lap_hi : P.dsdr2[it] / x2) : T(0);
+        if (c.magnetic && bot_radial) B[q0] = B[N + q0] = T(0);
+        if (c.magnetic && top_radial) B[q1] = B[N + q1] = T(0);
     }
 }
 
@@ -667,66 +682,53 @@ __global__ __launch_bounds__(256) void k_walls_density(Consts<T> c, Prof<T> P, W
                                                        const T *__restrict__ st, const T *__restrict__ B,
                                                        const T *__restrict__ D, const T *__restrict__ L,
                                                        int lbcr_rho, const T *__restrict__ tw, int theta) {
-    // theta = 0: the radial walls alone (k_rhs_line closes the theta walls itself)
+    // theta = 0: the radial walls alone (k_rhs_line closes the theta walls itself).  One thread per wall point, the
+    // four walls one after another: a thread that closed both ends of a pencil took the long chain of loads and
+    // terms twice (FP64 with explicit diffusion, 64x128x256: 53 us).
     const long nt = theta ? (long)c.nr * c.nphi : 0, nrr = (long)c.nth * c.nphi, N = c.N;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    // the momentum tendency before the density terms, evaluated at the wall points themselves
-    T o0[5], o1[5];
-    if (tw && i < nt) {
-        // the theta-wall block (k_walls_gather and the theta sweeps' end-row taps): the same
-        // values, one field after another with stride 2*nt
-        const int ir = (int)(i / c.nphi);
+    // the momentum tendency before the density terms, evaluated at the wall point itself
+    T o[5];
+    if (i < 2 * nt) {
+        const bool hi = i >= nt;
+        const long pencil = hi ? i - nt : i;   // (ip, ir)
+        const int ir = (int)(pencil / c.nphi), it = hi ? c.nth - 1 : 0;
         const T rv = P.r[ir] * c.invpconst;
-        Consts<T> cw = c;
-        cw.N = 2 * nt;
-        const T *stw = tw, *Bw = tw + 5 * cw.N, *Dw = tw + 8 * cw.N;
-        const long q0 = i, q1 = nt + i;
-        const Thermo<T> a0 = thermo(stw[q0], stw[4 * cw.N + q0], ir, cw, P);
-        const Thermo<T> a1 = thermo(stw[q1], stw[4 * cw.N + q1], ir, cw, P);
-        pre_density_terms(cw, P, stw, Bw, Dw, theta_from(Dw, cw.N, q0), L, q0, 0, ir, o0);
-        pre_density_terms(cw, P, stw, Bw, Dw, theta_from(Dw, cw.N, q1), L, q1, c.nth - 1, ir, o1);
-        wall[W.off_trho_lo + i] = rv * o0[1] * a0.rho / a0.t;
-        wall[W.off_trho_hi + i] = rv * o1[1] * a1.rho / a1.t;
-    } else if (i < nt) {
-        const int ir = (int)(i / c.nphi), ip = (int)(i % c.nphi);
-        const T rv = P.r[ir] * c.invpconst;
-        const long q0 = ((long)ir * c.nphi + ip) * c.nth, q1 = q0 + c.nth - 1;
-        const Thermo<T> a0 = thermo(st[q0], st[4 * N + q0], ir, c, P), a1 = thermo(st[q1], st[4 * N + q1], ir, c, P);
-        const T rho0 = a0.rho, rho1 = a1.rho, t0 = a0.t, t1 = a1.t;
-        pre_density_terms(c, P, st, B, D, theta_from(D, N, q0), L, q0, 0, ir, o0);
-        pre_density_terms(c, P, st, B, D, theta_from(D, N, q1), L, q1, c.nth - 1, ir, o1);
-        wall[W.off_trho_lo + i] = rv * o0[1] * rho0 / t0;
-        wall[W.off_trho_hi + i] = rv * o1[1] * rho1 / t1;
+        Thermo<T> a;
+        if (tw) {
+            // the theta-wall block (k_walls_gather and the theta sweeps' end-row taps): the same
+            // values, one field after another with stride 2*nt
+            Consts<T> cw = c;
+            cw.N = 2 * nt;
+            const T *stw = tw, *Bw = tw + 5 * cw.N, *Dw = tw + 8 * cw.N;
+            a = thermo(stw[i], stw[4 * cw.N + i], ir, cw, P);
+            pre_density_terms(cw, P, stw, Bw, Dw, theta_from(Dw, cw.N, i), L, i, it, ir, o);
+        } else {
+            const long q = pencil * c.nth + it;
+            a = thermo(st[q], st[4 * N + q], ir, c, P);
+            pre_density_terms(c, P, st, B, D, theta_from(D, N, q), L, q, it, ir, o);
+        }
+        wall[W.off_trho_lo + i] = rv * o[1] * a.rho / a.t;   // (the upper wall's values follow the lower one's)
+        return;
     }
-    if (i < nrr) {
-        const long q0 = i, q1 = (long)(c.nr - 1) * nrr + i;
-        const int it = (int)(i % c.nth);
-        const Thermo<T> a0 = thermo(st[q0], st[4 * N + q0], 0, c, P);
-        const Thermo<T> a1 = thermo(st[q1], st[4 * N + q1], c.nr - 1, c, P);
-        const T rho0 = a0.rho, rho1 = a1.rho, t0 = a0.t, t1 = a1.t;
-        const bool nlo = lbcr_rho == 2 || lbcr_rho == 4, nhi = lbcr_rho == 3 || lbcr_rho == 4;
-        T du0 = T(0), du1 = T(0);
-        if (nlo) {
-            pre_density_terms(c, P, st, B, D, theta_from(D, N, q0), L, q0, it, 0, o0);
-            du0 = o0[3];
-        }
-        if (nhi) {
-            pre_density_terms(c, P, st, B, D, theta_from(D, N, q1), L, q1, it, c.nr - 1, o1);
-            du1 = o1[3];
-        }
-        T lo = nlo ? du0 * rho0 * c.invpconst / t0 : rho0;
-        T hi = nhi ? du1 * rho1 * c.invpconst / t1 : rho1;
-        if (c.fluct) {
-            // the sweep differentiates rho - rho_bar, whose background derivative drbar already
-            // carries wbar at these walls: prescribe the departure
-            //   (du/dt without density terms + pconst (T_bar/rho_bar) wbar) rho/(pconst T) - wbar
-            //   = du_partial (rho/T)/pconst - wbar a/(1+a)      (du_partial: hres-based, small)
-            if (nlo) lo = du0 * (rho0 / t0) * c.invpconst - c.wbar_lo * a0.a / (T(1) + a0.a);
-            if (nhi) hi = du1 * (rho1 / t1) * c.invpconst - c.wbar_hi * a1.a / (T(1) + a1.a);
-        }
-        wall[W.off_rrho_lo + i] = lo / P.dxdr[0];
-        wall[W.off_rrho_hi + i] = hi / P.dxdr[c.nr - 1];
+    i -= 2 * nt;
+    if (i >= 2 * nrr) return;
+    const bool hi = i >= nrr;
+    const long pencil = hi ? i - nrr : i;   // (it, ip)
+    const int ir = hi ? c.nr - 1 : 0;
+    const long q = (long)ir * nrr + pencil;
+    const Thermo<T> a = thermo(st[q], st[4 * N + q], ir, c, P);
+    T val = a.rho;
+    if (hi ? lbcr_rho == 3 || lbcr_rho == 4 : lbcr_rho == 2 || lbcr_rho == 4) {
+        pre_density_terms(c, P, st, B, D, theta_from(D, N, q), L, q, (int)(pencil % c.nth), ir, o);
+        // in the fluctuation form the sweep differentiates rho - rho_bar, whose background derivative drbar
+        // already carries wbar at these walls: prescribe the departure
+        //   (du/dt without density terms + pconst (T_bar/rho_bar) wbar) rho/(pconst T) - wbar
+        //   = du_partial (rho/T)/pconst - wbar a/(1+a)      (du_partial: hres-based, small)
+        if (c.fluct) val = o[3] * (a.rho / a.t) * c.invpconst - (hi ? c.wbar_hi : c.wbar_lo) * a.a / (T(1) + a.a);
+        else val = o[3] * a.rho * c.invpconst / a.t;
     }
+    wall[W.off_rrho_lo + i] = val / P.dxdr[ir];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1242,6 +1244,28 @@ static int upload_profiles(cssx_mhd *m, Prof<T> &P) {
     const size_t o_eta = put(nr, [&](size_t i) { return opt(m->h_etar, i); });
     const size_t o_w9 = put(nr, [&](size_t i) { return opt(m->h_d2xdr2, i) / m->h_dxdr[i]; });
     const size_t o_d2s = put(nr, [&](size_t i) { return opt(m->h_d2sbar, i); });
+    // the compact operator's response to those wall derivatives: its rows with a one for the wall's value
+    std::vector<double> er[2];
+    for (int side = 0; side < 2; side++) {
+        const int bd = m->p.ibcr[1];
+        std::vector<double> l, u, &x = er[side];
+        x.assign(nr, 0.0);
+        if (side ? !(bd == 3 || bd == 4) : !(bd == 2 || bd == 4)) continue;
+        lhs_coefficients(1, nr, END_WALL, END_WALL, bd, l, u);
+        x[side ? nr - 1 : 0] = 1.0;
+        for (int j = 1; j < nr; j++) {   // u becomes the eliminated upper coefficient
+            const double piv = j > 1 ? 1.0 - l[j - 1] * u[j - 2] : 1.0;
+            u[j - 1] /= piv;
+            x[j - 1] = (x[j - 1] - (j > 1 ? l[j - 1] * x[j - 2] : 0.0)) / piv;
+        }
+        x[nr - 1] = (x[nr - 1] - l[nr - 1] * x[nr - 2]) / (1.0 - l[nr - 1] * u[nr - 2]);
+        for (int j = nr - 2; j >= 0; j--) x[j] -= u[j] * x[j + 1];
+        // below the rounding of the type it changes nothing
+        for (double &v : x)
+            if (std::fabs(v) < (f32 ? 1e-9 : 1e-18)) v = 0.0;
+    }
+    const size_t o_erl = put(nr, [&](size_t i) { return er[0][i] * m->h_dxdr[i]; });
+    const size_t o_erh = put(nr, [&](size_t i) { return er[1][i] * m->h_dxdr[i]; });
     const size_t tot = h.size();
     T *d = nullptr;
     if (P.buf) {
@@ -1259,6 +1283,7 @@ static int upload_profiles(cssx_mhd *m, Prof<T> &P) {
     P.rfc = d + o_rfc; P.rv = d + o_rv; P.sph = d + o_sph; P.rfac = d + o_rfac; P.ct = d + o_ct; P.gt = d + o_gt;
     P.vsp = d + o_vsp;
     P.mur = d + o_mur; P.dlnmu = d + o_dlm; P.ks = d + o_ks; P.dlnks = d + o_dlk; P.etar = d + o_eta;
+    P.erl = d + o_erl; P.erh = d + o_erh;
     P.w9 = d + o_w9; P.d2sbar = d + o_d2s;
     return CSSX_OK;
 }
@@ -1595,14 +1620,15 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
     const T *rho = st, *w = st + N, *v = st + 2 * N, *u = st + 3 * N, *s = st + 4 * N;
     const unsigned nb = nblocks(N, 256);
     // 1. B = curl A
-    if (m->p.magnetic && (rc = curl_impl<T>(m, st + 5 * N, B, stream))) return rc;
+    if (m->p.magnetic && (rc = curl_impl<T>(m, st + 5 * N, B, stream, false))) return rc;
     const T *bt = B, *bp = B + N, *br = B + 2 * N;
-    // 2. wall values
+    // 2. B on the walls, wall values
     {
         long nw = std::max((long)m->nr * m->nphi, (long)m->nth * m->nphi);
         hipLaunchKernelGGL(k_walls_state<T>, dim3(nblocks(nw, 256)), dim3(256), 0, stream, c, P, W, wall, st, B,
                            m->p.bottom_stress_free, m->p.top_stress_free, m->p.bottom_const_flux,
-                           m->p.top_const_flux, m->p.theta_normal_field);
+                           m->p.top_const_flux, m->p.theta_normal_field, m->p.theta_perf_cond, m->p.bottom_radial_field,
+                           m->p.top_radial_field);
     }
     // SLD diffusion of the stage-1 state: it needs only B and the state, and writes the SLD
     // tendency, its speed buffer and (RK4) the Ohmic curl, which nothing before the final kernel
@@ -1680,13 +1706,18 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
                            spec<T>(m, CSSX_AXIS_PHI, bt, D + D_PBT * N, 0, nullptr, nullptr),
                            spec<T>(m, CSSX_AXIS_PHI, br, D + D_PBR * N, 0, nullptr, nullptr)};
         if ((rc = derivs_axis<T>(m, CSSX_AXIS_PHI, ph, mag ? 7 : 5, stream))) return fail(rc);
-        DerivSpec rr[6] = {spec<T>(m, CSSX_AXIS_R, w, D + D_RW * N, ibcr[2], wall + W.off_rw_lo, wall + W.off_rw_hi, nullptr, P.dxdr),
+        DerivSpec rr[7] = {spec<T>(m, CSSX_AXIS_R, w, D + D_RW * N, ibcr[2], wall + W.off_rw_lo, wall + W.off_rw_hi, nullptr, P.dxdr),
                            spec<T>(m, CSSX_AXIS_R, v, D + D_RV * N, ibcr[3], wall + W.off_rv_lo, wall + W.off_rv_hi, nullptr, P.dxdr),
                            spec<T>(m, CSSX_AXIS_R, u, D + D_RU * N, ibcr[4], nullptr, nullptr, nullptr, P.dxdr),
-                           spec<T>(m, CSSX_AXIS_R, s, D + D_RS * N, ibcr[5], wall + W.off_rs_lo, wall + W.off_rs_hi, nullptr, P.dxdr),
-                           spec<T>(m, CSSX_AXIS_R, bt, D + D_RBT * N, ibcr[7], nullptr, nullptr, nullptr, P.dxdr),
-                           spec<T>(m, CSSX_AXIS_R, bp, D + D_RBP * N, ibcr[8], nullptr, nullptr, nullptr, P.dxdr)};
-        if ((rc = derivs_axis<T>(m, CSSX_AXIS_R, rr, mag ? 6 : 4, stream))) return fail(rc);
+                           spec<T>(m, CSSX_AXIS_R, s, D + D_RS * N, ibcr[5], wall + W.off_rs_lo, wall + W.off_rs_hi, nullptr, P.dxdr)};
+        int nrs = 4;
+        if (mag) {
+            rr[nrs++] = spec<T>(m, CSSX_AXIS_R, bt, D + D_RBT * N, ibcr[7], nullptr, nullptr, nullptr, P.dxdr);
+            rr[nrs++] = spec<T>(m, CSSX_AXIS_R, bp, D + D_RBP * N, ibcr[8], nullptr, nullptr, nullptr, P.dxdr);
+        }
+        // k_rhs_line adds what the density's wall derivatives, not known yet, contribute
+        if (line) rr[nrs++] = spec<T>(m, CSSX_AXIS_R, rho, D + D_RRHO * N, ibcr[1], nullptr, nullptr, nullptr, P.dxdr);
+        if ((rc = derivs_axis<T>(m, CSSX_AXIS_R, rr, nrs, stream))) return fail(rc);
     }
     // 3b. explicit diffusion: second derivatives (same wall values as the first), the cross-term
     //     sweeps of first-derivative slots, and curl B
@@ -1740,7 +1771,7 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
     // 4-5. density wall derivatives from the momentum tendency, which k_walls_density evaluates
     //      (every term before the density terms) at the wall points themselves
     {
-        const long nw = line ? (long)m->nth * m->nphi : std::max((long)m->nr * m->nphi, (long)m->nth * m->nphi);
+        const long nw = 2 * ((line ? 0 : (long)m->nr * m->nphi) + (long)m->nth * m->nphi);
         if (tw)
             hipLaunchKernelGGL(k_walls_gather<T>, dim3(nblocks((long)m->nr * m->nphi, 256)), dim3(256), 0, stream, c,
                                st, (const T *)B, (const T *)D, tw);
@@ -1754,7 +1785,7 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
         if (!line && (rc = derivs_axis<T>(m, CSSX_AXIS_THETA, &th, 1, stream))) return fail(rc);
         DerivSpec rr = spec<T>(m, CSSX_AXIS_R, rho, D + D_RRHO * N, ibcr[1], wall + W.off_rrho_lo,
                                wall + W.off_rrho_hi, nullptr, P.dxdr);
-        if ((rc = derivs_axis<T>(m, CSSX_AXIS_R, &rr, 1, stream))) return fail(rc);
+        if (!line && (rc = derivs_axis<T>(m, CSSX_AXIS_R, &rr, 1, stream))) return fail(rc);
         StageFuse<T> F0{};
         const StageFuse<T> &FF = F ? *F : F0;
         const float *ext = nullptr;
@@ -1786,6 +1817,7 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
             H.bw = ibct[2]; H.bv = ibct[3]; H.bu = ibct[4]; H.bs = ibct[5]; H.bbp = ibct[8]; H.bbr = ibct[9]; H.brho = ibct[1];
             H.tv_lo = wall + W.off_tv_lo; H.tv_hi = wall + W.off_tv_hi;
             H.tbp_lo = wall + W.off_tbp_lo; H.tbp_hi = wall + W.off_tbp_hi;
+            H.rr_lo = wall + W.off_rrho_lo; H.rr_hi = wall + W.off_rrho_hi;
             H.scale = (T)m->grid.dti;
             H.neu = (T)(1.0 / m->grid.dti);
             H.nl = lp.nl;

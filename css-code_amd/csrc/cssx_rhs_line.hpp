@@ -22,6 +22,7 @@ template <typename T>
 struct LineTheta {
     int bw, bv, bu, bs, bbp, bbr, brho;
     const T *tv_lo, *tv_hi, *tbp_lo, *tbp_hi;   // by pencil (ir * nphi + ip)
+    const T *rr_lo, *rr_hi;                     // the density's radial wall derivatives in x-space (nphi, nth)
     T scale, neu;
     // The strip: the workgroup's lanes from `off` on hold `pencils` pencils of nl lanes each; inv_nl = ceil(2^16 / nl)
     unsigned inv_nl;
@@ -192,6 +193,7 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
     const T ri = P.rinv[ir], rv = P.r[ir], epsr = P.eps[ir], g0 = FL ? P.hres[ir] : -P.grav[ir];
     const T rb = FL ? P.rbar[ir] : T(0), tbar = FL ? P.tbar[ir] : T(0), dsb = FL ? P.dsbar[ir] : T(0);
     const T tr = FL ? P.tr[ir] : T(0), drb = FL ? P.drbar[ir] : T(0);
+    const T erl = P.erl[ir], erh = P.erh[ir];
     const T omsq = rv * c.omega0 * c.omega0, om2 = c.om2;
     T cot[MR], sn[MR], cs[MR], csc[MR];
     theta(P.cot, cot);
@@ -365,6 +367,16 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
     }
     T drr[MR];
     field(dr_rho, drr);
+    // The r sweep of the density took zero wall derivatives, so that it runs with the other sweeps; theirs enter here,
+    // within their reach from the wall (48x96x96 FP32: one launch of 6.9 us less).
+    auto wall_part = [&](T e, const T *p) {
+        if (e != T(0)) {
+            run_load<T, MR, REM != 0>(p, ip0 * (unsigned)n + at, (long)c.nphi * n, x);
+            CSSX_K drr[k] = drr[k] + e * x[k];
+        }
+    };
+    wall_part(erl, H.rr_lo);
+    wall_part(erh, H.rr_hi);
     // ---- Density_Terms_Theta: the wall derivatives that zero the normal momentum tendency
     //      (rhs_mpi.f90:1553-1564), from the end points' own lanes
     {
