@@ -9,8 +9,8 @@
 //      :578-637)
 //   3. the 19 first-derivative sweeps of Source_Theta_Terms / Phi_Terms / Radial_Terms, batched
 //      per axis (one launch per axis, one job per field); with explicit diffusion also the 12
-//      second derivatives, the 6 cross-term sweeps of first-derivative slots and the 6 sweeps
-//      of curl B (Laplacian_Cross_Terms_*, VectorCurl)
+//      second derivatives, the 6 cross-term sweeps of first-derivative slots and the 3 or 4
+//      sweeps of curl B that are not among the first derivatives (Laplacian_Cross_Terms_*, VectorCurl)
 //   4. main_terms / viscous_terms: every pointwise term of those three routines in the
 //      reference's order, and the explicit-diffusion branches
 //   5. k_walls_density: the density wall derivatives that zero the normal momentum tendency
@@ -114,8 +114,8 @@ enum LapSlot {
     L_RW2, L_RV2, L_RU2, L_RS2,              // r second derivatives (x-space): w v u s
     L_XR1, L_XR2, L_XR3, L_XR4,              // cross terms: d/dr of dw/dth, du/dph, du/dth, dv/dph
     L_XT1, L_XT2,                            // cross terms: d/dth of dv/dph, dw/dph
-    L_JT1, L_JT2, L_JP1, L_JP2, L_JRT, L_JRP,  // curl B: d/dth (sin B_phi), d/dth B_r, d/dph B_r,
-                                             // d/dph B_theta, d/dr (r B_theta), d/dr (r B_phi)
+    L_JT1, L_JT2, L_JRT, L_JRP,              // curl B: d/dth (sin B_phi), d/dth B_r (with other theta walls than
+                                             // D_TBR's), d/dr (r B_theta), d/dr (r B_phi)
     L_NSLOT
 };
 
@@ -188,6 +188,7 @@ struct Consts {
     T gamm1, invtconst, invCv, pconst, invpconst, Cv, omega0, om2, xi2, gamma, T0, damp;
     int magnetic, top_relax, xi_on;
     int fluct;   // state slots 1 and 5 hold rho - rho_bar(r) and s - s_bar(r) (FP32 path)
+    int jt2;              // curl B takes d/dth B_r from L_JT2 instead of D_TBR
     int lap, slap;        // Laplacian; Laplacian or SLaplacian (thermal diffusion)
     T s_lap_lo, s_lap_hi; // constant-flux entropy wall values under slap: -lumr/(4 pi r^2 ks dxdr)
     T wbar_lo, wbar_hi;   // d rho_bar/dr prescribed at the Neumann density walls (0 elsewhere)
@@ -859,9 +860,9 @@ __device__ __forceinline__ void final_point(const Consts<T> &c, const Prof<T> &P
             // Induction_Terms with Laplacian (rhs_mpi.f90:2303-2322, VectorCurl derivatives.f90
             // :1894-2104): dA/dt -= etar curl B, ds/dt += (4 pi/c^2) etar |curl B|^2 / (rho T)
             const T ri = P.rinv[ir], csc = P.csc[it], eta = P.etar[ir];
-            const T jt = ri * L[L_JP1 * N + i] * csc - L[L_JRP * N + i] * ri;
-            const T jp = -L[L_JT2 * N + i] * ri + L[L_JRT * N + i] * ri;
-            const T jr = L[L_JT1 * N + i] * csc * ri - ri * L[L_JP2 * N + i] * csc;
+            const T jt = ri * D[D_PBR * N + i] * csc - L[L_JRP * N + i] * ri;
+            const T jp = -(c.jt2 ? L[L_JT2 * N + i] : td[D_TBR]) * ri + L[L_JRT * N + i] * ri;
+            const T jr = L[L_JT1 * N + i] * csc * ri - ri * D[D_PBT * N + i] * csc;
             da0 -= eta * jt;
             da1 -= eta * jp;
             da2 -= eta * jr;
@@ -1140,6 +1141,9 @@ __global__ __launch_bounds__(256) void k_cfl_final(const double *__restrict__ re
 // =============================================================================================
 namespace cssx {
 
+// closure of VectorCurl's theta sweeps: code 1 (Theta_Normal_Field) or 0, whose wall values go unused
+static int curl_b_theta_code(const cssx_mhd *m) { return m->p.theta_normal_field ? 1 : 0; }
+
 template <typename T>
 static Consts<T> make_consts(const cssx_mhd *m) {
     Consts<T> c;
@@ -1149,6 +1153,7 @@ static Consts<T> make_consts(const cssx_mhd *m) {
     c.xi2 = (T)(m->p.xi_cs * m->p.xi_cs); c.gamma = (T)m->p.gamma; c.T0 = (T)m->p.T0; c.damp = (T)m->p.damping_time;
     c.magnetic = m->p.magnetic; c.top_relax = m->p.top_relax; c.xi_on = m->p.xi_cs < 1.0;
     c.fluct = sizeof(T) == 4;
+    c.jt2 = curl_b_theta_code(m) != m->p.ibct[9];
     c.wbar_lo = (T)m->wbar_lo;
     c.wbar_hi = (T)m->wbar_hi;
     c.dT0top = m->h_tbar.empty() ? T(0) : (T)(m->p.T0 - m->h_tbar[m->nr - 1]);
@@ -1666,14 +1671,26 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
     T *tw = (!c.slap && !c.lap && !line) ? S.tw : nullptr;
     const long twM = 2L * m->nr * m->nphi;
     // 3. derivative sweeps
+    T *L = S.L;
     {
         const int mag = m->p.magnetic;
-        DerivSpec th[6] = {spec<T>(m, CSSX_AXIS_THETA, w, D + D_TW * N, ibct[2], nullptr, nullptr),
+        DerivSpec th[8] = {spec<T>(m, CSSX_AXIS_THETA, w, D + D_TW * N, ibct[2], nullptr, nullptr),
                            spec<T>(m, CSSX_AXIS_THETA, v, D + D_TV * N, ibct[3], wall + W.off_tv_lo, wall + W.off_tv_hi),
                            spec<T>(m, CSSX_AXIS_THETA, u, D + D_TU * N, ibct[4], nullptr, nullptr),
                            spec<T>(m, CSSX_AXIS_THETA, s, D + D_TS * N, ibct[5], nullptr, nullptr),
                            spec<T>(m, CSSX_AXIS_THETA, bp, D + D_TBP * N, ibct[8], wall + W.off_tbp_lo, wall + W.off_tbp_hi),
                            spec<T>(m, CSSX_AXIS_THETA, br, D + D_TBR * N, ibct[9], nullptr, nullptr)};
+        // curl B of the explicit diffusion (VectorCurl): theta sweeps of sin B_phi and, where its closure is another
+        // than D_TBR's, B_r; r sweeps of r B_theta and r B_phi with zero wall values (the radial-field walls zero
+        // those halos).  They need B alone and run with the other sweeps of their axis; the phi derivatives are
+        // D_PBR and D_PBT.  Six sweeps in three launches of their own: 64x128x256 FP64 680 -> 640 us.
+        const bool curl_b = mag && c.lap;
+        int nts = mag ? 6 : 4;
+        if (curl_b) {
+            const int tcode = curl_b_theta_code(m);
+            th[nts++] = spec<T>(m, CSSX_AXIS_THETA, bp, L + L_JT1 * N, tcode, nullptr, nullptr, P.sn);
+            if (c.jt2) th[nts++] = spec<T>(m, CSSX_AXIS_THETA, br, L + L_JT2 * N, tcode, nullptr, nullptr);
+        }
         if (tw) {
             // the theta sweeps copy their inputs and results at the theta-wall rows into the
             // theta-wall block (slots: w v u s -> 1..4, bp br -> B 1..2, results -> D slots)
@@ -1695,7 +1712,7 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
             for (DerivSpec &s : th) s.g_b *= m->nr - 1;
             if ((rc = run_derivs(th, mag ? 6 : 4, g, sizeof(T) == 8 ? CSSX_PREC_F64 : CSSX_PREC_F32, stream)))
                 return fail(rc);
-        } else if ((rc = derivs_axis<T>(m, CSSX_AXIS_THETA, th, mag ? 6 : 4, stream))) {
+        } else if ((rc = derivs_axis<T>(m, CSSX_AXIS_THETA, th, nts, stream))) {
             return fail(rc);
         }
         DerivSpec ph[7] = {spec<T>(m, CSSX_AXIS_PHI, rho, D + D_PRHO * N, 0, nullptr, nullptr),
@@ -1706,7 +1723,7 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
                            spec<T>(m, CSSX_AXIS_PHI, bt, D + D_PBT * N, 0, nullptr, nullptr),
                            spec<T>(m, CSSX_AXIS_PHI, br, D + D_PBR * N, 0, nullptr, nullptr)};
         if ((rc = derivs_axis<T>(m, CSSX_AXIS_PHI, ph, mag ? 7 : 5, stream))) return fail(rc);
-        DerivSpec rr[7] = {spec<T>(m, CSSX_AXIS_R, w, D + D_RW * N, ibcr[2], wall + W.off_rw_lo, wall + W.off_rw_hi, nullptr, P.dxdr),
+        DerivSpec rr[8] = {spec<T>(m, CSSX_AXIS_R, w, D + D_RW * N, ibcr[2], wall + W.off_rw_lo, wall + W.off_rw_hi, nullptr, P.dxdr),
                            spec<T>(m, CSSX_AXIS_R, v, D + D_RV * N, ibcr[3], wall + W.off_rv_lo, wall + W.off_rv_hi, nullptr, P.dxdr),
                            spec<T>(m, CSSX_AXIS_R, u, D + D_RU * N, ibcr[4], nullptr, nullptr, nullptr, P.dxdr),
                            spec<T>(m, CSSX_AXIS_R, s, D + D_RS * N, ibcr[5], wall + W.off_rs_lo, wall + W.off_rs_hi, nullptr, P.dxdr)};
@@ -1715,13 +1732,16 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
             rr[nrs++] = spec<T>(m, CSSX_AXIS_R, bt, D + D_RBT * N, ibcr[7], nullptr, nullptr, nullptr, P.dxdr);
             rr[nrs++] = spec<T>(m, CSSX_AXIS_R, bp, D + D_RBP * N, ibcr[8], nullptr, nullptr, nullptr, P.dxdr);
         }
+        if (curl_b) {
+            rr[nrs++] = spec<T>(m, CSSX_AXIS_R, bt, L + L_JRT * N, ibcr[7], nullptr, nullptr, P.r, P.dxdr);
+            rr[nrs++] = spec<T>(m, CSSX_AXIS_R, bp, L + L_JRP * N, ibcr[8], nullptr, nullptr, P.r, P.dxdr);
+        }
         // k_rhs_line adds what the density's wall derivatives, not known yet, contribute
         if (line) rr[nrs++] = spec<T>(m, CSSX_AXIS_R, rho, D + D_RRHO * N, ibcr[1], nullptr, nullptr, nullptr, P.dxdr);
         if ((rc = derivs_axis<T>(m, CSSX_AXIS_R, rr, nrs, stream))) return fail(rc);
     }
     // 3b. explicit diffusion: second derivatives (same wall values as the first), the cross-term
     //     sweeps of first-derivative slots, and curl B
-    T *L = S.L;
     if (c.slap) {
         const int nd = c.lap ? 4 : 1;
         DerivSpec th[4] = {spec2<T>(m, CSSX_AXIS_THETA, s, L + L_TS2 * N, ibct[5], nullptr, nullptr),
@@ -1753,20 +1773,6 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
         DerivSpec xt[2] = {spec<T>(m, CSSX_AXIS_THETA, D + D_PV * N, L + L_XT1 * N, ibct[3], lw + 2 * nrr, lw + 2 * nrr + nt),
                            spec<T>(m, CSSX_AXIS_THETA, D + D_PW * N, L + L_XT2 * N, ibct[2], nullptr, nullptr)};
         if ((rc = derivs_axis<T>(m, CSSX_AXIS_THETA, xt, 2, stream))) return fail(rc);
-        if (m->p.magnetic) {
-            // VectorCurl: theta sweeps with code 1 (Theta_Normal_Field) or 0, whose wall values go
-            // unused; r sweeps with zero wall values (the radial-field walls zero those halos)
-            const int tcode = m->p.theta_normal_field ? 1 : 0;
-            DerivSpec jt[2] = {spec<T>(m, CSSX_AXIS_THETA, bp, L + L_JT1 * N, tcode, nullptr, nullptr, P.sn),
-                               spec<T>(m, CSSX_AXIS_THETA, br, L + L_JT2 * N, tcode, nullptr, nullptr)};
-            if ((rc = derivs_axis<T>(m, CSSX_AXIS_THETA, jt, 2, stream))) return fail(rc);
-            DerivSpec jp[2] = {spec<T>(m, CSSX_AXIS_PHI, br, L + L_JP1 * N, 0, nullptr, nullptr),
-                               spec<T>(m, CSSX_AXIS_PHI, bt, L + L_JP2 * N, 0, nullptr, nullptr)};
-            if ((rc = derivs_axis<T>(m, CSSX_AXIS_PHI, jp, 2, stream))) return fail(rc);
-            DerivSpec jr[2] = {spec<T>(m, CSSX_AXIS_R, bt, L + L_JRT * N, ibcr[7], nullptr, nullptr, P.r, P.dxdr),
-                               spec<T>(m, CSSX_AXIS_R, bp, L + L_JRP * N, ibcr[8], nullptr, nullptr, P.r, P.dxdr)};
-            if ((rc = derivs_axis<T>(m, CSSX_AXIS_R, jr, 2, stream))) return fail(rc);
-        }
     }
     // 4-5. density wall derivatives from the momentum tendency, which k_walls_density evaluates
     //      (every term before the density terms) at the wall points themselves
@@ -1798,11 +1804,11 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
             if (rc) return fail(rc);
             ext = m->ext;
         }
-        // reads: 5 state, 3 B, 19 (13) first-derivative and 2 density-derivative fields, 18 (3)
+        // reads: 5 state, 3 B, 19 (13) first-derivative and 2 density-derivative fields, 15 (3)
         // explicit-diffusion fields with Laplacian (SLaplacian); the plain RHS writes 8 (5)
         // tendencies, a fused stage moves the stage traffic of every field instead
         const bool mag = m->p.magnetic;
-        const double reads = (mag ? 29.0 : 20.0) - (line ? (mag ? 7.0 : 5.0) : 0.0) + (c.lap ? 18.0 : c.slap ? 3.0 : 0.0);
+        const double reads = (mag ? 29.0 : 20.0) - (line ? (mag ? 7.0 : 5.0) : 0.0) + (c.lap ? 15.0 : c.slap ? 3.0 : 0.0);
         const double fb = !F ? (mag ? 8.0 : 5.0) * sizeof(T)
                           : sizeof(T) == 8 ? (FF.stage == 1 ? 24.0 + (FF.dif ? 8.0 : 0.0) : FF.stage < 4 ? 32.0 : 24.0) * m->nv
                                            : (FF.stage == 1 ? 12.0 + (FF.dif ? 4.0 : 0.0) : FF.stage < 4 ? 16.0 : 24.0) * m->nv;
