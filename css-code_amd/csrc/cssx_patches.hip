@@ -1,5 +1,5 @@
-// Batched compact derivatives of many independent patches of uneven shape in one persistent
-// launch (gfx950).  Each patch is a small subdomain f(nth, nphi, nr) with walls on all six
+// Batched compact derivatives of many independent patches of uneven shape in one launch
+// (gfx950).  Each patch is a small subdomain f(nth, nphi, nr) with walls on all six
 // faces (the Dbydr/Dbydt/Dbydp closures of derivatives.f90:547-796, :1010-1262 applied on
 // every axis, as Determine_Dtype's dtype 0 would ask); all three first derivatives of every
 // patch are work items of one kernel:
@@ -9,8 +9,12 @@
 // both with the constant-coefficient recurrences of cssx_uniform.hpp: an item reads no plan, a seg_item
 // exchanges its carries at two barriers and a line_item has none.  Pencils too short for them (fewer than
 // 32 rows in FP32, 48 in FP64) run on the plan-driven strided_item / contig_item.
-// Workgroups loop over the item table (persistent, as many as can be resident).  (MR, NT) are template
-// choices; cssx_patchset_autotune times the instantiated variants on the actual patch set.
+// One workgroup per item.  As many workgroups as are resident at once, each looping over the table, ran in step: all
+// loading, then all storing; started one by one as others end they spread out.  16 patches of 32..512 points per
+// axis in FP32: 3284 -> 2791 us (8 rows per lane of a theta item), 3238 -> 2494 (16 rows; 5.0 TB/s); sets of 8 to 12
+// smaller ones 294 -> 277 and 289 -> 266, in FP64 621 -> 584 and 620 -> 553 (8 rows), 636 -> 610 and 615 -> 579 (16).
+// (MR, NT) are template choices: a set starts with the faster of those, 16 rows in FP32 and 8 in FP64, and
+// cssx_patchset_autotune times the instantiated variants on the actual patch set.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -179,7 +183,6 @@ __device__ __forceinline__ void strided_item(const PatchJob<T> &J, int ablk, int
         const T x = (jj < mi) ? d[jj] + vL[pst + jj] * xl + vR[pst + jj] * xr : xr;
         bstore(J.scale * x, rout, o0 + (unsigned)jj * rowb, 0u);
     }
-    __syncthreads();   // LDS reused by the next item
 }
 
 template <typename T, int MR, int NT>
@@ -283,7 +286,6 @@ __device__ __forceinline__ void contig_item(const PatchJob<T> &J, int ablk, int 
 #pragma unroll
         for (int jj = 0; jj < MR; jj++) bstore(d[jj], rout, jj < m ? o0 + (unsigned)(jj * sizeof(T)) : kNoPencil, 0u);
     }
-    __syncthreads();   // LDS reused by the next item
 }
 
 // S segments of the columns [blk*P, +P) (the recurrences and exchanges of k_deriv_seg)
@@ -441,33 +443,29 @@ __device__ __forceinline__ void line_item(const PatchJob<T> &J, int blk) {
 // FP32 is held to 64 VGPRs: eight waves per SIMD (two 1024-lane or four 512-lane workgroups per CU)
 template <typename T, int MR, int NT>
 __global__ __launch_bounds__(NT, (sizeof(T) == 4 && MR == 8) ? 8 : 1) void k_patch_derivs(const PatchJob<T> *__restrict__ jobs,
-                                                       const int4 *__restrict__ items, int nitems) {
+                                                       const int4 *__restrict__ items) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T *sp = reinterpret_cast<T *>(smem_raw);
-    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
-        const int4 w = items[xcd_neighbour(it, nitems)];
-        const PatchJob<T> &J = jobs[w.x];
-        if (J.kind == PK_LINE) {
-            line_item<T, MR, NT>(J, w.y);
-        } else if (J.kind == PK_SEG) {
-            if constexpr (sizeof(T) == 4) {
-                switch (J.M) {
-                case 20: seg_item<T, 20, NT>(J, w.y, sp); break;
-                case 24: seg_item<T, 24, NT>(J, w.y, sp); break;
-                case 28: seg_item<T, 28, NT>(J, w.y, sp); break;
-                default: seg_item<T, 32, NT>(J, w.y, sp); break;
-                }
-            } else {
-                if (J.M == 12) seg_item<T, 12, NT>(J, w.y, sp);
-                else seg_item<T, 16, NT>(J, w.y, sp);
+    const int4 w = items[xcd_neighbour(blockIdx.x, gridDim.x)];
+    const PatchJob<T> &J = jobs[w.x];
+    if (J.kind == PK_LINE) {
+        line_item<T, MR, NT>(J, w.y);
+    } else if (J.kind == PK_SEG) {
+        if constexpr (sizeof(T) == 4) {
+            switch (J.M) {
+            case 20: seg_item<T, 20, NT>(J, w.y, sp); break;
+            case 24: seg_item<T, 24, NT>(J, w.y, sp); break;
+            case 28: seg_item<T, 28, NT>(J, w.y, sp); break;
+            default: seg_item<T, 32, NT>(J, w.y, sp); break;
             }
-        } else if (J.kind == PK_STRIDED) {
-            __syncthreads();   // a seg_item before it may still be reading its exchange arrays
-            strided_item<T, 16, NT>(J, w.y, w.z, sp);
         } else {
-            __syncthreads();
-            contig_item<T, 8, NT>(J, w.y, w.z, sp);
+            if (J.M == 12) seg_item<T, 12, NT>(J, w.y, sp);
+            else seg_item<T, 16, NT>(J, w.y, sp);
         }
+    } else if (J.kind == PK_STRIDED) {
+        strided_item<T, 16, NT>(J, w.y, w.z, sp);
+    } else {
+        contig_item<T, 8, NT>(J, w.y, w.z, sp);
     }
 }
 
@@ -672,17 +670,9 @@ hipError_t launch_variant(const cssx_patchset *ps, int var, hipStream_t s) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
     }
-    int dev = 0, ncu = 256, per_cu = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    // persistent grid: as many workgroups as can be resident at once, so none waits for another
-    // to drain the item list
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, NT, shm);
-    if (e != hipSuccess) return e;
-    const long g = std::min<long>(ps->nitems[var], (long)ncu * std::max(1, per_cu));
-    if (g < 1) return hipSuccess;
-    hipLaunchKernelGGL((k_patch_derivs<T, MR, NT>), dim3((unsigned)g), dim3(NT), shm, s,
-                       (const PatchJob<T> *)ps->jobs[var], (const int4 *)ps->items[var], (int)ps->nitems[var]);
+    if (ps->nitems[var] < 1) return hipSuccess;
+    hipLaunchKernelGGL((k_patch_derivs<T, MR, NT>), dim3((unsigned)ps->nitems[var]), dim3(NT), shm, s,
+                       (const PatchJob<T> *)ps->jobs[var], (const int4 *)ps->items[var]);
     return hipGetLastError();
 }
 
@@ -723,6 +713,7 @@ extern "C" int cssx_patchset_create(const cssx_patch *patches, int npatch, int p
     if (!ps) return CSSX_ENOMEM;
     ps->prec = prec;
     ps->npatch = npatch;
+    ps->best = prec == CSSX_PREC_F32 ? 2 : 0;
     for (int v = 0; v < kPatchVariants; v++) {
         int rc = prec == CSSX_PREC_F64 ? build_variant<double>(ps, patches, v) : build_variant<float>(ps, patches, v);
         if (rc) {

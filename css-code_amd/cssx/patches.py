@@ -1,7 +1,7 @@
 """Batched derivatives of many uneven patches (cssx_patchset) and the ensemble of small MHD runs.
 
 A patch is an independent subdomain f(nth, nphi, nr) with walls on all six faces; all three
-first derivatives of every patch of a set run as one persistent launch (csrc/cssx_patches.hip).
+first derivatives of every patch of a set run as one launch (csrc/cssx_patches.hip).
 `patch_shapes` draws the lengths (uniform integers in [lo, hi] per axis from the project's
 SplitMix64 generator), `PatchChunk` owns the device memory of a set of patches (one arena per
 role, every patch 256-byte aligned), fills it with seeded smoothed noise and runs / autotunes
@@ -32,7 +32,7 @@ def patch_shapes(count: int, seed: int = 4, lo: int = 32, hi: int = 512):
 
 
 class PatchChunk:
-    """Device buffers, patch table and persistent-launch plan for a list of patch shapes."""
+    """Device buffers, patch and item tables for a list of patch shapes."""
 
     def __init__(self, shapes, prec: str = "f32", bdry: int = 1, axes=(True, True, True), device="cuda"):
         if not torch.cuda.is_available():

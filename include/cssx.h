@@ -248,7 +248,7 @@ int cssx_plan_tables(int n, int order, int lo_kind, int hi_kind, int bdry, int v
 /* ---- batched patches ---------------------------------------------------------------------------
  * Many independent subdomains ("patches") of uneven shape f(nth, nphi, nr), each with walls on
  * all six faces (the wall closures of derivatives.f90 with boundary code bdry on every axis,
- * prescribed wall derivatives zero), differentiated along r, theta and phi in ONE persistent
+ * prescribed wall derivatives zero), differentiated along r, theta and phi in ONE
  * launch per cssx_patchset_run.  Pencil lengths 8..512.  Outputs that are NULL are skipped.
  * Results are in index units times dri/dti/dpi, as cssx_deriv's. */
 typedef struct cssx_patch {
@@ -265,7 +265,7 @@ typedef struct cssx_patchset cssx_patchset;
  * bytes (the kernels' 32-bit buffer offsets) */
 int cssx_patchset_create(const cssx_patch *patches, int npatch, int prec, cssx_patchset **out);
 void cssx_patchset_destroy(cssx_patchset *ps);
-/* one persistent launch over every item; variant -1 = the autotuned (or default) one */
+/* one launch over every item; variant -1 = the autotuned (or default) one */
 int cssx_patchset_run(cssx_patchset *ps, int variant, void *stream);
 /* times each variant (reps runs), keeps the fastest; synchronizes.  ms_out (4 floats) may be NULL */
 int cssx_patchset_autotune(cssx_patchset *ps, int reps, void *stream, int *best, float *ms_out);
