@@ -27,6 +27,7 @@ struct LineTheta {
     // The strip: the workgroup's lanes from `off` on hold `pencils` pencils of nl lanes each; inv_nl = ceil(2^16 / nl)
     unsigned inv_nl;
     int nl, pencils, off;
+    int near_xcd;   // neighbouring workgroups on one XCD (xcd_neighbour)
 };
 
 // k / w for w = 3 or 6 (rw = 1/w), rounded as the division is: the remainder of k rw is exact, and adding its
@@ -138,8 +139,14 @@ __device__ __forceinline__ void rhs_line(const Consts<T> &c, const Prof<T> &P, c
     const int lane = threadIdx.x & 63, s0 = (int)threadIdx.x - H.off;
     const int pl = s0 < 0 ? H.pencils : (int)((unsigned)s0 * H.inv_nl >> 16);
     constexpr bool FL = sizeof(T) == 4;   // fluctuation form (Consts::fluct)
-    const unsigned ip0 = blockIdx.x * (unsigned)H.pencils;
-    const int ir = (int)blockIdx.y;
+    unsigned bx = blockIdx.x;
+    int ir = (int)blockIdx.y;
+    if (H.near_xcd) {   // (the last workgroup stays the last)
+        const unsigned i = xcd_neighbour(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+        ir = (int)(i / gridDim.x);
+        bx = i - (unsigned)ir * gridDim.x;
+    }
+    const unsigned ip0 = bx * (unsigned)H.pencils;
     const unsigned id0 = (unsigned)ir * (unsigned)c.nphi + ip0;
     const bool active = pl < H.pencils && ip0 + pl < (unsigned)c.nphi;
     // lanes without a pencil work along on the first one and store nothing
