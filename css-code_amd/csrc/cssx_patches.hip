@@ -670,10 +670,16 @@ hipError_t launch_variant(const cssx_patchset *ps, int var, hipStream_t s) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
     }
-    if (ps->nitems[var] < 1) return hipSuccess;
-    hipLaunchKernelGGL((k_patch_derivs<T, MR, NT>), dim3((unsigned)ps->nitems[var]), dim3(NT), shm, s,
-                       (const PatchJob<T> *)ps->jobs[var], (const int4 *)ps->items[var]);
-    return hipGetLastError();
+    // A launch counts its work-items in 32 bits, and one of more starts without an error but short of what the count
+    // wraps by: a set of 2^22 items at 1024 lanes to a workgroup, or 2^23 at 512, takes more than one.
+    const long n = ps->nitems[var], most = 0xffffffffL / NT;
+    for (long at = 0; at < n; at += most) {
+        hipLaunchKernelGGL((k_patch_derivs<T, MR, NT>), dim3((unsigned)std::min(most, n - at)), dim3(NT), shm, s,
+                           (const PatchJob<T> *)ps->jobs[var], (const int4 *)ps->items[var] + at);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <typename T>

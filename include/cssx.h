@@ -249,7 +249,8 @@ int cssx_plan_tables(int n, int order, int lo_kind, int hi_kind, int bdry, int v
  * Many independent subdomains ("patches") of uneven shape f(nth, nphi, nr), each with walls on
  * all six faces (the wall closures of derivatives.f90 with boundary code bdry on every axis,
  * prescribed wall derivatives zero), differentiated along r, theta and phi in ONE
- * launch per cssx_patchset_run.  Pencil lengths 8..512.  Outputs that are NULL are skipped.
+ * launch per cssx_patchset_run (more only beyond 2^32 work-items: millions of small items).
+ * Pencil lengths 8..512.  Outputs that are NULL are skipped.
  * Results are in index units times dri/dti/dpi, as cssx_deriv's. */
 typedef struct cssx_patch {
     int nr, nth, nphi;
