@@ -107,12 +107,15 @@ static int uniform_min(bool f64) { return f64 ? 48 : 32; }
 // Whether a launch runs on the constant-coefficient kernels: walls at both ends (unit-stride pencils in
 // planes that lie back to back or apart, or strided ones) or the periodic wrap (strided), of enough rows, with
 // nothing asked for but f' (the assembled rows of compact_fd6 and its halo ends stay with the plan-driven kernels).
-static bool use_uniform(const DerivSpec *sp, int nspec, const AxisGeom &g, bool f64) {
+static bool uniform_geom(const AxisGeom &g, bool f64) {
     if (g.n < uniform_min(f64) || g.n > 1024) return false;
-    const bool unit = g.srow == 1;
+    if (g.srow == 1) return g.sa == g.n && (g.nb <= 1 || g.sb >= (long)g.n * g.na);
     int M, G, S;
-    if (!unit && !seg_shape(g.n, f64, 0, 1, M, G, S)) return false;
-    if (unit && (g.sa != g.n || (g.nb > 1 && g.sb < (long)g.n * g.na))) return false;
+    return seg_shape(g.n, f64, 0, 1, M, G, S) && seg_span_fits(g.n, g.na, g.nb, g.sa, g.sb, g.srow, f64 ? 8 : 4);
+}
+static bool use_uniform(const DerivSpec *sp, int nspec, const AxisGeom &g, bool f64) {
+    if (!uniform_geom(g, f64)) return false;
+    const bool unit = g.srow == 1;
     for (int i = 0; i < nspec; i++) {
         const DerivSpec &s = sp[i];
         const bool wall = s.lo_kind == END_WALL && s.hi_kind == END_WALL;
@@ -281,6 +284,8 @@ extern "C" int cssx_ctx_create(const cssx_grid *grid, cssx_ctx **out) {
     }
     // build every plan this grid can ask for, so that later calls do not allocate
     int ns[3] = {grid->nr, grid->nth, grid->nphi};
+    AxisGeom geom[3];
+    for (int ax = 0; ax < 3; ax++) axis_geometry(ax, grid->nth, grid->nphi, grid->nr, geom[ax]);
     for (int ax = 0; ax < 3; ax++)
         for (int order = 1; order <= 2; order++)
             for (int lo = 0; lo < 2; lo++)
@@ -290,10 +295,7 @@ extern "C" int cssx_ctx_create(const cssx_grid *grid, cssx_ctx **out) {
                         if (lo == 1 && hi == 1 && bd > 0) continue;
                         // walls at both ends: no plan where the constant-coefficient kernels serve both
                         // precisions
-                        int sM, sG, sS;
-                        if (lo == 0 && hi == 0 && ns[ax] >= uniform_min(true) &&
-                            (ax == CSSX_AXIS_THETA || (seg_shape(ns[ax], true, 0, 1, sM, sG, sS) && seg_shape(ns[ax], false, 0, 1, sM, sG, sS))))
-                            continue;
+                        if (lo == 0 && hi == 0 && uniform_geom(geom[ax], true) && uniform_geom(geom[ax], false)) continue;
                         PlanKey key{ns[ax], order, lo ? END_HALO : END_WALL, hi ? END_HALO : END_WALL, bd};
                         const void *p;
                         for (int var = 0; var < 2; var++) {

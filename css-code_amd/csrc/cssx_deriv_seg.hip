@@ -14,6 +14,8 @@
 // pencil, with no exchange at all, measured 216 and 212 us there but 46 against 32 us at 128x256x512.)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "cssx_bufio.hpp"
 #include "cssx_plan.hpp"
 #include "cssx_uniform.hpp"
@@ -334,13 +336,23 @@ bool seg_shape(int n, bool f64, long cols, int njobs, int &M, int &G, int &S) {
     return found;
 }
 
+// Whether a lane's rows lie within 32-bit byte offsets of its block's first slow index.  A block's up to 64 columns run
+// over the end of the fast index: t slow indices on, its last lane is at fast index na + 62 - t * na at most.
+bool seg_span_fits(int n, int na, int nb, long sa, long sb, long srow, size_t elem) {
+    double span = 0.0;
+    for (int t = 0; t < nb && (long)t * na <= na + 62L; t++) {
+        const long a = t == 0 ? na - 1L : std::min(na - 1L, na + 62L - (long)t * na);
+        span = std::max(span, (double)t * (double)sb + (double)a * (double)sa);
+    }
+    return (span + (double)(n - 1) * (double)srow + 1.0) * (double)elem < 4294967295.0;
+}
+
 template <typename T>
 hipError_t launch_deriv_seg(const DerivLaunch<T> &L0, int order, hipStream_t stream) {
     DerivLaunch<T> L = L0;
     int M, G, S;
     if (!seg_shape(L.n, sizeof(T) == 8, (long)L.na * L.nb, L.njobs, M, G, S) || L.njobs < 1 || L.njobs > kMaxJobs || L.n < 32)
         return hipErrorInvalidValue;
-    // 32-bit byte offsets of a lane: columns of up to 64 / na + 2 slow indices
     const int P = 64 / G;
     bool flat = L.nb > 1 && L.sa == 1 && L.sb == L.na;
     for (int i = 0; i < L.njobs; i++) {
@@ -349,9 +361,7 @@ hipError_t launch_deriv_seg(const DerivLaunch<T> &L0, int order, hipStream_t str
     }
     // (a field past the 32-bit offsets keeps its slow index in the base pointer)
     flat = flat && ((double)L.na * L.nb + (double)(L.n - 1) * L.srow) * sizeof(T) < 4294967295.0;
-    const double slow = flat ? 0.0 : (double)(P / L.na + 1) * (double)L.sb;
-    const double span = flat ? (double)L.na * L.nb : (double)(L.na - 1) * L.sa + 1.0;
-    if ((slow + span + (double)(L.n - 1) * L.srow) * sizeof(T) >= 4294967295.0) return hipErrorInvalidValue;
+    if (!flat && !seg_span_fits(L.n, L.na, L.nb, L.sa, L.sb, L.srow, sizeof(T))) return hipErrorInvalidValue;
     if (flat) {   // the two pencil indices are one contiguous run
         L.na = L.na * L.nb;
         L.nb = 1;

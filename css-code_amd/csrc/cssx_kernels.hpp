@@ -56,6 +56,8 @@ template <typename T>
 hipError_t launch_deriv_seg(const DerivLaunch<T> &L, int order, hipStream_t stream);
 // the segmentation of that kernel for a launch of njobs fields of `cols` columns; false: n has none
 bool seg_shape(int n, bool f64, long cols, int njobs, int &M, int &G, int &S);
+// whether that kernel's 32-bit byte offsets hold the launch
+bool seg_span_fits(int n, int na, int nb, long sa, long sb, long srow, size_t elem);
 // walls at both ends, unit row stride, same lengths (L.M rows per lane, L.S lanes per pencil)
 template <typename T>
 hipError_t launch_deriv_line(const DerivLaunch<T> &L, int order, hipStream_t stream);
