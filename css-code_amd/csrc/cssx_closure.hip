@@ -25,6 +25,7 @@
 #include <mutex>
 #include <new>
 #include <set>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -499,6 +500,7 @@ __global__ __launch_bounds__(512) void k_closure_infer(const T *__restrict__ st,
 // fields lie in two 16-byte quarters, as the tables' do, instead of 24 four-byte reads per K step.
 // 64x128x256 FP32: one tile at a time 540 us, two 437, with gelu2 423 (448 TFLOP/s; the vector ALU's share
 // alone is 375); the next pair's footprints asked for before the products: 436.
+// NU tiles at a time (closure_tendency chooses).
 constexpr int kFoot = 8 * 3 * 3 * 18;   // footprint values per tile
 constexpr int kInferWaves = 8;
 constexpr size_t kInferRowsBytes = kPackBytes + 2 * kFeat * sizeof(float) + (size_t)kInferWaves * kFoot * sizeof(float);
@@ -509,7 +511,7 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <typename T>
+template <typename T, int NU>
 __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
     const T *__restrict__ st, long N, int nr, int nphi, int nth, int fluct, const T *__restrict__ rbar,
     const T *__restrict__ sbar, const float *__restrict__ xmean, const float *__restrict__ xistd,
@@ -601,29 +603,33 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
             b[ks] = __builtin_bit_cast(cssx_bf16x8, w);
         }
     };
-    const long step = 2L * gridDim.x * kInferWaves;
-    long t = 2 * ((long)blockIdx.x * kInferWaves + wv);
+    const long step = (long)NU * gridDim.x * kInferWaves;
+    long t = NU * ((long)blockIdx.x * kInferWaves + wv);
     for (; t < ntiles; t += step) {
-        const bool two = t + 1 < ntiles;   // else the second half repeats the last tile and stores nothing
+        const bool two = NU == 2 && t + 1 < ntiles;   // else a second half repeats the last tile and stores nothing
         // one lane address per array, taken anew for each pair (constant offsets from there): kept across the loop
         // the addresses and the values behind them would not fit the registers
         int fresh = 0;
         asm volatile("" : "+s"(fresh));
         const cssx_bf16 *w1 = W1T + (li * kS1 + 8 * g + fresh), *w2 = W2P + (li * kS2 + 8 * g + fresh);
         const cssx_bf16 *w3 = W3P + (li * kS2 + 8 * g + fresh);
-        cssx_bf16x8 b[2][kKp1 / 32];
-        T raw[2][24];
+        cssx_bf16x8 b[NU][kKp1 / 32];
+        T raw[NU][24];
         fetch(t, raw[0]);
-        fetch(two ? t + 1 : t, raw[1]);
+        if constexpr (NU == 2) fetch(two ? t + 1 : t, raw[1]);
         features(t, raw[0], b[0]);
         __builtin_amdgcn_sched_barrier(0);
-        features(two ? t + 1 : t, raw[1], b[1]);
-        __builtin_amdgcn_sched_barrier(0);
-        cssx_f32x4 acc[2][8];
-        cssx_bf16x8 h[2][4];
+        if constexpr (NU == 2) {
+            features(two ? t + 1 : t, raw[1], b[1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        cssx_f32x4 acc[NU][8];
+        cssx_bf16x8 h[NU][4];
         auto clear = [&]() {
 #pragma unroll
-            for (int nb = 0; nb < 8; nb++) acc[0][nb] = acc[1][nb] = cssx_f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int u = 0; u < NU; u++)
+#pragma unroll
+                for (int nb = 0; nb < 8; nb++) acc[u][nb] = cssx_f32x4{0.f, 0.f, 0.f, 0.f};
         };
         auto activate = [&](const float *bias) __attribute__((always_inline)) {
 #pragma unroll
@@ -631,7 +637,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
                 const float4 bb = *reinterpret_cast<const float4 *>(bias + nb * 16);
                 const float bv[4] = {bb.x, bb.y, bb.z, bb.w};
 #pragma unroll
-                for (int u = 0; u < 2; u++)
+                for (int u = 0; u < NU; u++)
 #pragma unroll
                     for (int r = 0; r < 4; r++) h[u][nb >> 1][(nb & 1) * 4 + r] = (cssx_bf16)gelu2(acc[u][nb][r] + bv[r]);
             }
@@ -643,7 +649,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
             for (int nb = 0; nb < 8; nb++) {
                 const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(w1 + nb * 16 * kS1 + ks * 32);
 #pragma unroll
-                for (int u = 0; u < 2; u++) acc[u][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[u][ks], acc[u][nb], 0, 0, 0);
+                for (int u = 0; u < NU; u++) acc[u][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[u][ks], acc[u][nb], 0, 0, 0);
             }
         __builtin_amdgcn_sched_barrier(0);
         activate(b1 + (4 * g + fresh));
@@ -655,17 +661,17 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
             for (int nb = 0; nb < 8; nb++) {
                 const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(w2 + nb * 16 * kS2 + ks * 32);
 #pragma unroll
-                for (int u = 0; u < 2; u++) acc[u][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[u][ks], acc[u][nb], 0, 0, 0);
+                for (int u = 0; u < NU; u++) acc[u][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[u][ks], acc[u][nb], 0, 0, 0);
             }
         __builtin_amdgcn_sched_barrier(0);
         activate(b2 + (4 * g + fresh));
         __builtin_amdgcn_sched_barrier(0);
-        cssx_f32x4 y[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        cssx_f32x4 y[NU] = {};
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
             const cssx_bf16x8 a = *reinterpret_cast<const cssx_bf16x8 *>(w3 + ks * 32);
 #pragma unroll
-            for (int u = 0; u < 2; u++) y[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[u][ks], y[u], 0, 0, 0);
+            for (int u = 0; u < NU; u++) y[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, h[u][ks], y[u], 0, 0, 0);
         }
         if (g < 2) {
             const int o = 4 * g + fresh;
@@ -674,7 +680,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_closure_infer_rows(
                 float *e = ext + ((long)(o + r) * N + t * 16 + li);
                 const float sc = ystd[o + r], of = ymean[o + r], bo = b3[o + r];
                 e[0] = (y[0][r] + bo) * sc + of;
-                if (two) e[16] = (y[1][r] + bo) * sc + of;
+                if (two) e[16] = (y[NU - 1][r] + bo) * sc + of;
             }
         }
     }
@@ -849,7 +855,7 @@ int fused_setup(const void *fn, size_t lds, int *ncu) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return CSSX_EHIP;
     std::lock_guard<std::mutex> lk(mu);
-    if (!raised.count({fn, dev})) {
+    if (fn && !raised.count({fn, dev})) {
         if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
             return CSSX_EHIP;
         raised.insert({fn, dev});
@@ -877,19 +883,25 @@ int closure_tendency(cssx_mlp *n, int prec, const void *st, int fluct, const voi
         if (nth % 16 == 0 && 8.0 * (double)N * (prec == CSSX_PREC_F64 ? 8.0 : 4.0) < 4294967295.0) {
             // tiles of 16 points inside one theta row (and 32-bit byte offsets over the 8 fields): the
             // footprint-staged kernel
-            const void *fr = prec == CSSX_PREC_F64 ? (const void *)k_closure_infer_rows<double>
-                                                   : (const void *)k_closure_infer_rows<float>;
-            if (int rc = fused_setup(fr, kInferRowsBytes, &ncu)) return rc;
-            const unsigned grid = (unsigned)std::min<long>((long)ncu, (tiles + 2 * kInferWaves - 1) / (2 * kInferWaves));
+            auto rows = [&](auto prec_tag, auto nu) -> int {
+                using T = decltype(prec_tag);
+                constexpr int NU = decltype(nu)::value;
+                if (int rc = fused_setup((const void *)k_closure_infer_rows<T, NU>, kInferRowsBytes, &ncu)) return rc;
+                const unsigned grid = (unsigned)std::min<long>((long)ncu, (tiles + NU * kInferWaves - 1) / (NU * kInferWaves));
+                hipLaunchKernelGGL((k_closure_infer_rows<T, NU>), dim3(grid), dim3(64 * kInferWaves), kInferRowsBytes, s,
+                                   (const T *)st, N, nr, nphi, nth, fluct, (const T *)rbar, (const T *)sbar, n->xmean,
+                                   n->xistd, n->ymean, n->ystd, n->pk, ext);
+                return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
+            };
+            if (int rc = fused_setup(nullptr, 0, &ncu)) return rc;   // the CU count alone
+            // A pass of pairs takes 12.3 us and one of single tiles 7.5 (FP64 states: 13.5 and 8.0), so pairs are taken
+            // where they save enough passes: with 256 CUs, pairs against single tiles, whole call in FP32: 2048 tiles
+            // 22.1 / 17.0 us, 4096 22.5 / 25.7, 6144 34.5 / 32.1, 8192 34.8 / 42.6, 10240 48.2 / 50.7.
+            const long once = (long)ncu * kInferWaves;   // tiles in flight, one per wavefront
+            const bool pairs = 2 * ((tiles + once - 1) / once) > 3 * ((tiles + 2 * once - 1) / (2 * once));
             if (prec == CSSX_PREC_F64)
-                hipLaunchKernelGGL(k_closure_infer_rows<double>, dim3(grid), dim3(64 * kInferWaves), kInferRowsBytes, s,
-                                   (const double *)st, N, nr, nphi, nth, fluct, (const double *)rbar,
-                                   (const double *)sbar, n->xmean, n->xistd, n->ymean, n->ystd, n->pk, ext);
-            else
-                hipLaunchKernelGGL(k_closure_infer_rows<float>, dim3(grid), dim3(64 * kInferWaves), kInferRowsBytes, s,
-                                   (const float *)st, N, nr, nphi, nth, fluct, (const float *)rbar,
-                                   (const float *)sbar, n->xmean, n->xistd, n->ymean, n->ystd, n->pk, ext);
-            return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
+                return pairs ? rows(double{}, std::integral_constant<int, 2>{}) : rows(double{}, std::integral_constant<int, 1>{});
+            return pairs ? rows(float{}, std::integral_constant<int, 2>{}) : rows(float{}, std::integral_constant<int, 1>{});
         }
         const void *fn = prec == CSSX_PREC_F64 ? (const void *)k_closure_infer<double> : (const void *)k_closure_infer<float>;
         if (int rc = fused_setup(fn, kPackBytes, &ncu)) return rc;
