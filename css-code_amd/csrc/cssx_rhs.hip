@@ -119,6 +119,12 @@ enum LapSlot {
     L_NSLOT
 };
 
+// How k_rhs_line lays the theta pencils of nth rows over a workgroup's lanes
+struct LinePlan {
+    int waves = 0, nl = 0, pencils = 0, off = 0;   // waves = 0: the sweeps and k_rhs_final serve the size
+    bool cut = false;                              // a pencil spans two wavefronts
+};
+
 template <typename T>
 struct Scratch {
     T *D = nullptr;      // D_NSLOT fields
@@ -136,6 +142,7 @@ struct Scratch {
     T *y0f = nullptr;    // FP32 runs: the FP64 state y0 in stage precision, fluctuation form
     T *L = nullptr;      // explicit diffusion: L_NSLOT fields
     T *lwall = nullptr;  // explicit diffusion: cross-term wall values (2 r, 2 theta buffers)
+    LinePlan line;       // of k_rhs_line, searched once (cssx_mhd_create): a search takes up to 30 us of host time
     bool ready = false;
 };
 
@@ -1398,11 +1405,6 @@ static bool sld_fork_ok(cssx_mhd *m, hipStream_t stream) {
     return true;
 }
 
-// How k_rhs_line lays the theta pencils of nth rows over a workgroup's lanes
-struct LinePlan {
-    int waves = 0, nl = 0, pencils = 0, off = 0;   // waves = 0: the sweeps and k_rhs_final serve the size
-    bool cut = false;                              // a pencil spans two wavefronts
-};
 template <typename T>
 constexpr int line_run() { return 4; }   // rows per lane (k_rhs_line)
 // The strip of 1, 2 or 4 wavefronts that leaves the fewest lanes idle; pencils cut by a wavefront's end
@@ -1666,7 +1668,7 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
     };
     // the theta-wall block for the density wall closure: without explicit diffusion (whose
     // viscous terms the closure would read too)
-    const LinePlan lp = line_plan<T>(m);
+    const LinePlan &lp = S.line;
     const bool line = lp.waves > 0;
     T *tw = (!c.slap && !c.lap && !line) ? S.tw : nullptr;
     const long twM = 2L * m->nr * m->nphi;
@@ -2130,6 +2132,8 @@ extern "C" int cssx_mhd_create(const cssx_grid *grid, const cssx_mhd_params *par
     }
     m->dth = (m->h_theta[nth - 1] - m->h_theta[0]) / (nth - 1);
     m->dphi = 1.0 / grid->dpi;
+    m->s64.line = line_plan<double>(m);
+    m->s32.line = line_plan<float>(m);
     m->h_tbar.resize(nr);
     for (int i = 0; i < nr; i++)
         m->h_tbar[i] = m->invtconst * std::pow(m->h_rho_bar[i], m->gamm1) * std::exp(m->h_s_bar[i] * m->invCv);
