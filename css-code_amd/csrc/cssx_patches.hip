@@ -13,7 +13,7 @@
 // loading, then all storing; started one by one as others end they spread out.  16 patches of 32..512 points per
 // axis in FP32: 3284 -> 2791 us (8 rows per lane of a theta item), 3238 -> 2494 (16 rows; 5.0 TB/s); sets of 8 to 12
 // smaller ones 294 -> 277 and 289 -> 266, in FP64 621 -> 584 and 620 -> 553 (8 rows), 636 -> 610 and 615 -> 579 (16).
-// (MR, NT) are template choices: a set starts with the faster of those, 16 rows in FP32 and 8 in FP64, and
+// (MR, NT) are template choices: start_variant picks the one a set starts with, and
 // cssx_patchset_autotune times the instantiated variants on the actual patch set.
 #include <hip/hip_runtime.h>
 
@@ -562,7 +562,7 @@ extern "C" int cssx_patch_fill(void *out, void *tmp, int prec, int nr, int nth, 
 
 struct cssx_patchset {
     int prec = 0, npatch = 0, nmax_short = 0, best = 0;   // nmax_short: longest plan-driven pencil
-    long nitems[kPatchVariants] = {};
+    long nitems[kPatchVariants] = {}, nplan[kPatchVariants] = {};   // items; the plan-driven ones among them
     void *jobs[kPatchVariants] = {};
     int4 *items[kPatchVariants] = {};
 };
@@ -643,6 +643,7 @@ int build_variant(cssx_patchset *ps, const cssx_patch *pt, int var) {
                 const long p = J.kind == PK_CONTIG ? (long)(NT / 64) * (64 / J.lanes) : NT / J.lanes;
                 per_b = (J.na + p - 1) / p;
                 ps->nmax_short = std::max(ps->nmax_short, J.n);
+                ps->nplan[var] += per_b * nb;
             }
             const int jid = (int)jobs.size();
             jobs.push_back(J);
@@ -660,6 +661,18 @@ int build_variant(cssx_patchset *ps, const cssx_patch *pt, int var) {
                                    hipMemcpyHostToDevice) != hipSuccess))
         return CSSX_EHIP;
     return CSSX_OK;
+}
+
+// The variant a set starts with.  1024 lanes to a workgroup, and the faster run length of each type (above); 512 lanes
+// where more than three quarters of the items are plan-driven: those cover the pencils of one plane each and leave
+// most of a large workgroup idle.  1024 -> 512 lanes (8 rows per lane) in FP32 / FP64: 256 patches of 16^3 169 -> 69 / 328 -> 133
+// us, 64 of 8..31 points per axis 45 -> 23 / 101 -> 41, 60 of 8x8x512 294 -> 154 / 743 -> 304 (plan-driven items
+// only), 300 of 32..64 719 -> 425 (FP64, 79% of the items), 4 of 500x20x500 96 -> 93 (FP32, 76%); with fewer it is the other
+// way round: 4 of 500x20x500 218 -> 226 (FP64, 61%), 4 of 20x500x500 90 -> 93 / 211 -> 217 (52% / 35%), 24 of
+// 32..256 324 -> 353 / 692 -> 737 (0 / 1%).
+int start_variant(const cssx_patchset *ps) {
+    const int v = ps->prec == CSSX_PREC_F32 ? 2 : 0;
+    return 4 * ps->nplan[v] > 3 * ps->nitems[v] ? 1 : v;
 }
 
 template <typename T, int MR, int NT>
@@ -719,7 +732,6 @@ extern "C" int cssx_patchset_create(const cssx_patch *patches, int npatch, int p
     if (!ps) return CSSX_ENOMEM;
     ps->prec = prec;
     ps->npatch = npatch;
-    ps->best = prec == CSSX_PREC_F32 ? 2 : 0;
     for (int v = 0; v < kPatchVariants; v++) {
         int rc = prec == CSSX_PREC_F64 ? build_variant<double>(ps, patches, v) : build_variant<float>(ps, patches, v);
         if (rc) {
@@ -727,6 +739,7 @@ extern "C" int cssx_patchset_create(const cssx_patch *patches, int npatch, int p
             return rc;
         }
     }
+    ps->best = start_variant(ps);
     *out = ps;
     return CSSX_OK;
 }
