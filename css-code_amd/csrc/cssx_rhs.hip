@@ -1832,10 +1832,12 @@ static int rhs_body(cssx_mhd *m, const T *st, T *dv, T *Bout, hipStream_t stream
             H.pencils = lp.pencils;
             H.off = lp.off;
             // Neighbouring workgroups on one XCD, which then works in an eighth of the window that the launch has
-            // open in each of its 50 to 60 streams (fewer pages to translate, most likely: only very large fields gain).  RK4 step,
-            // dealt round-robin against this: 256x512x1024 FP32 (537 MB a field) 52.0 -> 49.9 ms, FP64 101.0 -> 99.0,
-            // 200x400x700 FP64 (448 MB) 45.6 -> 45.4; 256x512x600 FP32 (315 MB) 29.3 -> 29.4, 128x256x512 FP64 (134 MB) 11.98 ->
-            // 12.14, FP32 (67 MB) 6.53 -> 6.78.
+            // open in each of its 50 to 60 streams (fewer pages to translate, most likely).  RK4 step without SLD, dealt
+            // round-robin against this, best of three processes (which differ by up to 8%): FP32 256x512x1024 (537 MB a
+            // field) 41.8 -> 38.5 ms, 400x251x1000 (402 MB) 34.1 -> 33.0, 300x500x700 (420 MB) 34.7 -> 33.4; FP64
+            // 256x256x1024 (537 MB) 38.7 -> 37.0; 256x512x1024, 200x400x700 and 300x480x600 in FP64, 320x400x1000,
+            // 500x352x640, 200x1024x512 and 390x257x1023 in FP32 (410 to 1074 MB) within 1% either way.  Smaller fields lose:
+            // 256x512x600 FP32 (315 MB) 29.3 -> 29.4, 128x256x512 FP64 (134 MB) 11.98 -> 12.14, FP32 (67 MB) 6.53 -> 6.78.
             H.near_xcd = (double)N * sizeof(T) >= 4e8;
             H.inv_nl = (65536u + lp.nl - 1) / lp.nl;
             CSSX_TIMED(CSSX_PHASE_RHS_FINAL, stream, bytes,
