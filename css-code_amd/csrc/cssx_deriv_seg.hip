@@ -103,7 +103,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(G == 1 ? 8
         if (lo) {
             const T val = (pen_ok && J.glo) ? J.glo[gbase] * J.neu_mul : T(0);
             const T e[6] = {w[2], w[3], w[4], w[5], w[6], w[7]};
-            wall_rhs<T, ORDER, false>(e, bd, val, J.lo_r0_val != 0, scale, r0, r1);
+            wall_rhs<T, ORDER, false>(e, bd, val, scale, r0, r1);
         }
         if (hi) {
             const T val = (pen_ok && J.ghi) ? J.ghi[gbase] * J.neu_mul : T(0);
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(G == 1 ? 8
 #pragma unroll
                 for (int s = 1; s < TAIL; s++) e[t] = m == M - s ? w[M + 1 - t - s] : e[t];
             }
-            wall_rhs<T, ORDER, true>(e, bd, val, false, scale, q0, q1);
+            wall_rhs<T, ORDER, true>(e, bd, val, scale, q0, q1);
         }
     } else {
         // periodic: the seam rows take the neighbour's derivative from the explicit formula

@@ -175,13 +175,13 @@ __device__ __forceinline__ T line_solve(const LineShape<MR, REM> &G, T (&v)[MR],
     T r0 = T(0), r1 = T(0), q0 = T(0), q1 = T(0);
     {
         const T e[6] = {f(0), f(1), f(2), f(3), f(4), f(5)};
-        wall_rhs<T, ORDER, false>(e, bd, lo_val, false, scale, r0, r1);
+        wall_rhs<T, ORDER, false>(e, bd, lo_val, scale, r0, r1);
     }
 #pragma unroll
     for (int k = 0; k < MR; k++)
         if (k == kn2) {
             const T e[6] = {f(k + 1), f(k), f(k - 1), f(k - 2), f(k - 3), f(k - 4)};
-            wall_rhs<T, ORDER, true>(e, bd, hi_val, false, scale, q0, q1);
+            wall_rhs<T, ORDER, true>(e, bd, hi_val, scale, q0, q1);
         }
     // ---- forward: rows 0, 1 and n-2, n-1 are not uniform rows and stay zero
     const Stencil<T, ORDER> S(scale);

@@ -327,7 +327,7 @@ __device__ __forceinline__ void seg_item(const PatchJob<T> &J, int blk, T *sp) {
     T r0 = T(0), r1 = T(0), q0 = T(0), q1 = T(0);
     if (lo) {
         const T e[6] = {w[2], w[3], w[4], w[5], w[6], w[7]};
-        wall_rhs<T, 1, false>(e, bd, T(0), false, scale, r0, r1);
+        wall_rhs<T, 1, false>(e, bd, T(0), scale, r0, r1);
     }
     if (hi) {
         T e[6];   // row n-1 sits at w[m + 1]
@@ -337,7 +337,7 @@ __device__ __forceinline__ void seg_item(const PatchJob<T> &J, int blk, T *sp) {
 #pragma unroll
             for (int s = 1; s < TAIL; s++) e[t] = m == M - s ? w[M + 1 - t - s] : e[t];
         }
-        wall_rhs<T, 1, true>(e, bd, T(0), false, scale, q0, q1);
+        wall_rhs<T, 1, true>(e, bd, T(0), scale, q0, q1);
     }
     const Stencil<T, 1> St(scale);
     const int me = hi ? m - 2 : m;

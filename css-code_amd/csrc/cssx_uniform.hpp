@@ -14,8 +14,13 @@
 //
 // A pencil cut into segments solves each with zero carry-in; a carry Y from below adds
 // (-a)^(j+1) Y to row j and a carry X from above (-a)^(m-j) X.  a = 0.382 (first derivative) and 0.188
-// (second): a carry is below the rounding of the type (a^reach < 2^-28, 2^-55) `reach` rows on, so it
+// (second): a carry is below an eighth of the rounding of the type (a^reach < 2^-27, 2^-55) `reach` rows on, so it
 // spans the next one to few segments only and needs no reduced system.
+//
+// What that means for results: an error is small against the largest value within `reach` rows or so, not against
+// a much smaller value there (the tail of a spike ends about `reach` rows from it instead of decaying on), and a NaN or
+// an infinity fills that reach and the rest of the segments or lanes it meets (up to 55 rows either way in FP32, 81 in
+// FP64), not the whole pencil.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -38,15 +43,19 @@ struct Uni<2> {
     static constexpr double l1 = 0.1, u1 = -0.35;
     static constexpr int reach32 = 12, reach64 = 24;
 };
-// rows after which a carry is below the rounding of T
-template <typename T, int ORDER>
-constexpr int uni_reach() { return sizeof(T) == 4 ? Uni<ORDER>::reach32 : Uni<ORDER>::reach64; }
 // (-a)^k
 template <int ORDER>
 __host__ __device__ constexpr double uni_pow(int k) {
     double v = 1.0;
     for (int i = 0; i < (k < 0 ? -k : k); i++) v *= -Uni<ORDER>::a;
     return k < 0 ? 1.0 / v : v;
+}
+// rows after which a carry is below the rounding of T
+template <typename T, int ORDER>
+constexpr int uni_reach() {
+    constexpr int r = sizeof(T) == 4 ? Uni<ORDER>::reach32 : Uni<ORDER>::reach64;
+    static_assert(r % 2 == 0 && uni_pow<ORDER>(r) < (sizeof(T) == 4 ? 0x1p-27 : 0x1p-55), "a carry is cut too early");
+    return r;
 }
 // The first wall row's coefficient of x_1 (cssx_plan.cpp lhs_coefficients) and the reciprocal of the
 // eliminated wall system's pivot, by closure kind; compile-time constants, selected per launch.
@@ -60,12 +69,12 @@ struct UniWall {
 // right-hand sides of the two wall rows at the lower (HI = false) or upper end, f[k] the k-th point from
 // the wall, val the prescribed wall derivative in index units; times `scale`
 template <typename T, int ORDER, bool HI>
-__device__ __forceinline__ void wall_rhs(const T (&f)[6], int bd, T val, bool r0_val, T scale, T &r0, T &r1) {
+__device__ __forceinline__ void wall_rhs(const T (&f)[6], int bd, T val, T scale, T &r0, T &r1) {
     const bool dirichlet = HI ? (bd == 1 || bd == 2) : (bd == 1 || bd == 3);
     if constexpr (ORDER == 1) {
         const T s1 = Rows<T, 1>::wall1(f[0], f[1], f[2], f[3], f[4]);
         const T s0 = Rows<T, 1>::wall0(dirichlet, (HI ? (bd == 3 || bd == 4) : bd != 0) ? val : T(0), f[0], f[1], f[2],
-                                       f[3], s1, r0_val);
+                                       f[3], s1);
         r1 = HI ? -s1 : s1;
         r0 = (HI && dirichlet) ? -s0 : s0;
     } else {

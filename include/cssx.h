@@ -70,7 +70,11 @@ void cssx_ctx_destroy(cssx_ctx *ctx);
  *             At a physical wall slot 0 holds the prescribed physical first derivative
  *             (NULL = 0).  On phi, NULL ghosts select the single-subdomain periodic wrap.
  * The result is f' (or f'') in index units times dri/dti/dpi (squared for order 2), exactly
- * what the reference returns; the caller multiplies by dx/dr on a stretched radial grid. */
+ * what the reference returns; the caller multiplies by dx/dr on a stretched radial grid.
+ * Pencils of 48 rows on (FP32: 32) between two walls, or on phi's wrap, are solved by recurrences that end some 20
+ * (FP32) or 40 (FP64) rows from where they start: errors are relative to the largest value in that reach, and a NaN or
+ * infinity fills that reach and the rest of the segments it meets (up to 55 / 81 rows either way), not the whole
+ * pencil. */
 int cssx_deriv(cssx_ctx *ctx, int axis, int order, int bdry, int prec, const void *in, void *out,
                const void *ghost_lo, const void *ghost_hi, void *stream);
 
