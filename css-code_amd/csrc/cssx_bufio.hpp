@@ -65,6 +65,17 @@ __device__ __forceinline__ unsigned xcd_neighbour(unsigned i, unsigned n) {
     return g + 128u <= n ? g + (r & 7u) * 16u + (r >> 3) : i;
 }
 
+// Elementwise launches over n items, 256 to a workgroup: rows of at most 2^23 workgroups, because a launch counts the
+// work-items of each dimension in 32 bits and wraps without an error.
+inline dim3 item_grid(long n) {
+    constexpr long row = 1L << 23;
+    const long wgs = (n + 255) / 256;
+    return dim3((unsigned)(wgs < row ? wgs : row), (unsigned)((wgs + row - 1) / row));
+}
+__device__ __forceinline__ long item_index() {
+    return ((long)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+}
+
 // v from lane l of the wavefront as a wave-uniform value (v_readlane)
 __device__ __forceinline__ float lane_val(float v, int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));

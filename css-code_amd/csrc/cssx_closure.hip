@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256) void k_box_filter(const Tin *__restrict__ in, 
                                                     int nr, int nphi, int nth, int f) {
     const int cr = nr / f, cp = nphi / f, ct = nth / f;
     const long Nc = (long)cr * cp * ct;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = item_index();
     if (i >= Nc * nv) return;
     const int iv = (int)(i / Nc);
     long j = i - (long)iv * Nc;
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void k_features(const T *__restrict__ st, long
                                                   long row0, long rows, const float *__restrict__ mean,
                                                   const float *__restrict__ istd, cssx_bf16 *__restrict__ xb,
                                                   float *__restrict__ xf) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = item_index();
     if (e >= rows * kFeat) return;
     const long pt = row0 + e / kFeat;
     const int q = (int)(e - (e / kFeat) * kFeat);
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float *__restrict__ p, cs
 __global__ __launch_bounds__(256) void k_add_closure(const float *__restrict__ Y, long rows, long row0, long N,
                                                      const float *__restrict__ ymean, const float *__restrict__ ystd,
                                                      float *__restrict__ ext) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = item_index();
     if (e >= rows * kOut) return;
     const long r = e / kOut;
     const int iv = (int)(e - r * kOut);
@@ -274,7 +274,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_targets(const float *__restrict__ fine, const T *__restrict__ coarse, long N,
                                                  const float *__restrict__ ymean, const float *__restrict__ ystd,
                                                  float *__restrict__ out, float *__restrict__ raw) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = item_index();
     if (e >= N * kOut) return;
     const long r = e / kOut;
     const int iv = (int)(e - r * kOut);
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(256) void k_field_stats(const T *__restrict__ st, i
 // dst[i] = src[idx[i]] for rows of rowbytes bytes (a multiple of 4)
 __global__ __launch_bounds__(256) void k_gather_rows(const unsigned *__restrict__ src, const long *__restrict__ idx,
                                                      long n, int words, unsigned *__restrict__ dst) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = item_index();
     if (e >= n * words) return;
     const long r = e / words;
     const int w = (int)(e - r * words);
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(256) void k_gather_rows(const unsigned *__restrict_
 __global__ __launch_bounds__(256) void k_standardize(const float *__restrict__ x, long rows, int cols,
                                                      const float *__restrict__ mean, const float *__restrict__ sd,
                                                      cssx_bf16 *__restrict__ ob, float *__restrict__ of) {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long e = item_index();
     if (e >= rows * cols) return;
     const int c = (int)(e % cols);
     const float v = (x[e] - mean[c]) / sd[c];
@@ -836,7 +836,7 @@ int mlp_backward(cssx_mlp *n, const cssx_bf16 *X, const float *Tg, int rows, hip
 template <typename T>
 int features_impl(cssx_mlp *n, const T *st, long N, int nr, int nphi, int nth, int fluct, const T *rbar,
                   const T *sbar, long row0, long rows, cssx_bf16 *xb, float *xf, hipStream_t s) {
-    hipLaunchKernelGGL(k_features<T>, dim3(nblk(rows * kFeat)), dim3(256), 0, s, st, N, nr, nphi, nth, fluct, rbar,
+    hipLaunchKernelGGL(k_features<T>, item_grid(rows * kFeat), dim3(256), 0, s, st, N, nr, nphi, nth, fluct, rbar,
                        sbar, row0, rows, n ? n->xmean : nullptr, n ? n->xistd : nullptr, xb, xf);
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
@@ -925,7 +925,7 @@ int closure_tendency(cssx_mlp *n, int prec, const void *st, int fluct, const voi
                                             (const float *)sbar, r0, rows, n->X, nullptr, s);
         if (rc) return rc;
         if ((rc = mlp_forward(n, n->X, (int)rows, false, s))) return rc;
-        hipLaunchKernelGGL(k_add_closure, dim3(nblk(rows * kOut)), dim3(256), 0, s, n->Y, rows, r0, N, n->ymean,
+        hipLaunchKernelGGL(k_add_closure, item_grid(rows * kOut), dim3(256), 0, s, n->Y, rows, r0, N, n->ymean,
                            n->ystd, ext);
     }
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
@@ -1110,10 +1110,10 @@ extern "C" int cssx_box_filter(const void *in, int prec, int nv, int nr, int nph
     const long Nc = (long)(nr / factor) * (nphi / factor) * (nth / factor) * nv;
     hipStream_t s = (hipStream_t)stream;
     if (prec == CSSX_PREC_F64)
-        hipLaunchKernelGGL(k_box_filter<double>, dim3(nblk(Nc)), dim3(256), 0, s, (const double *)in, out, nv, nr, nphi,
+        hipLaunchKernelGGL(k_box_filter<double>, item_grid(Nc), dim3(256), 0, s, (const double *)in, out, nv, nr, nphi,
                            nth, factor);
     else
-        hipLaunchKernelGGL(k_box_filter<float>, dim3(nblk(Nc)), dim3(256), 0, s, (const float *)in, out, nv, nr, nphi,
+        hipLaunchKernelGGL(k_box_filter<float>, item_grid(Nc), dim3(256), 0, s, (const float *)in, out, nv, nr, nphi,
                            nth, factor);
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
@@ -1140,10 +1140,10 @@ extern "C" int cssx_closure_targets(const float *fine_filtered, const void *coar
         return CSSX_EINVAL;
     hipStream_t s = (hipStream_t)stream;
     if (prec == CSSX_PREC_F64)
-        hipLaunchKernelGGL(k_targets<double>, dim3(nblk(npts * kOut)), dim3(256), 0, s, fine_filtered,
+        hipLaunchKernelGGL(k_targets<double>, item_grid(npts * kOut), dim3(256), 0, s, fine_filtered,
                            (const double *)coarse_rhs, npts, y_mean, y_std, target, raw);
     else
-        hipLaunchKernelGGL(k_targets<float>, dim3(nblk(npts * kOut)), dim3(256), 0, s, fine_filtered,
+        hipLaunchKernelGGL(k_targets<float>, item_grid(npts * kOut), dim3(256), 0, s, fine_filtered,
                            (const float *)coarse_rhs, npts, y_mean, y_std, target, raw);
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
@@ -1207,7 +1207,7 @@ extern "C" int cssx_field_stats(const void *state, int prec, int nv, int nr, int
 extern "C" int cssx_gather_rows(const void *src, long row_bytes, const long *idx, long n, void *dst, void *stream) {
     if (!src || !idx || !dst || n < 1 || row_bytes < 4 || row_bytes % 4) return CSSX_EINVAL;
     const int words = (int)(row_bytes / 4);
-    hipLaunchKernelGGL(k_gather_rows, dim3(nblk(n * words)), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(k_gather_rows, item_grid(n * words), dim3(256), 0, (hipStream_t)stream,
                        (const unsigned *)src, idx, n, words, (unsigned *)dst);
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
@@ -1215,7 +1215,7 @@ extern "C" int cssx_gather_rows(const void *src, long row_bytes, const long *idx
 extern "C" int cssx_standardize_rows(const float *x, long rows, int cols, const float *mean, const float *stddev,
                                      void *out_bf16, float *out_f32, void *stream) {
     if (!x || rows < 1 || cols < 1 || !mean || !stddev || (!out_bf16 && !out_f32)) return CSSX_EINVAL;
-    hipLaunchKernelGGL(k_standardize, dim3(nblk(rows * cols)), dim3(256), 0, (hipStream_t)stream, x, rows, cols, mean,
+    hipLaunchKernelGGL(k_standardize, item_grid(rows * cols), dim3(256), 0, (hipStream_t)stream, x, rows, cols, mean,
                        stddev, (cssx_bf16 *)out_bf16, out_f32);
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }

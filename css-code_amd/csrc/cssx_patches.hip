@@ -500,7 +500,7 @@ __device__ __forceinline__ double splitmix_u01(unsigned long long seed, unsigned
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_patch_noise(T *out, long n, unsigned long long seed) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = item_index();
     if (i >= n) return;
     const long m = (n + 1) / 2, k = i >> 1;
     const double u1 = splitmix_u01(seed, (unsigned long long)k), u2 = splitmix_u01(seed, (unsigned long long)(m + k));
@@ -528,12 +528,11 @@ using namespace cssx;
 
 extern "C" int cssx_normal_fill(void *out, int prec, long n, unsigned long long seed, void *stream) {
     if (!out || n < 1 || (prec != CSSX_PREC_F64 && prec != CSSX_PREC_F32)) return CSSX_EINVAL;
-    const unsigned g = (unsigned)((n + 255) / 256);
     hipStream_t s = (hipStream_t)stream;
     if (prec == CSSX_PREC_F64)
-        hipLaunchKernelGGL(k_patch_noise<double>, dim3(g), dim3(256), 0, s, (double *)out, n, seed);
+        hipLaunchKernelGGL(k_patch_noise<double>, item_grid(n), dim3(256), 0, s, (double *)out, n, seed);
     else
-        hipLaunchKernelGGL(k_patch_noise<float>, dim3(g), dim3(256), 0, s, (float *)out, n, seed);
+        hipLaunchKernelGGL(k_patch_noise<float>, item_grid(n), dim3(256), 0, s, (float *)out, n, seed);
     return hipGetLastError() == hipSuccess ? CSSX_OK : CSSX_EHIP;
 }
 
@@ -546,13 +545,13 @@ extern "C" int cssx_patch_fill(void *out, void *tmp, int prec, int nr, int nth, 
     hipStream_t s = (hipStream_t)stream;
     if (prec == CSSX_PREC_F64) {
         double *o = (double *)out, *t = (double *)tmp;
-        hipLaunchKernelGGL(k_patch_noise<double>, dim3(g), dim3(256), 0, s, t, n, seed);
+        hipLaunchKernelGGL(k_patch_noise<double>, item_grid(n), dim3(256), 0, s, t, n, seed);
         hipLaunchKernelGGL(k_patch_smooth<double>, dim3(g), dim3(256), 0, s, t, o, n, 1L, nth);
         hipLaunchKernelGGL(k_patch_smooth<double>, dim3(g), dim3(256), 0, s, o, t, n, (long)nth, nphi);
         hipLaunchKernelGGL(k_patch_smooth<double>, dim3(g), dim3(256), 0, s, t, o, n, (long)nth * nphi, nr);
     } else {
         float *o = (float *)out, *t = (float *)tmp;
-        hipLaunchKernelGGL(k_patch_noise<float>, dim3(g), dim3(256), 0, s, t, n, seed);
+        hipLaunchKernelGGL(k_patch_noise<float>, item_grid(n), dim3(256), 0, s, t, n, seed);
         hipLaunchKernelGGL(k_patch_smooth<float>, dim3(g), dim3(256), 0, s, t, o, n, 1L, nth);
         hipLaunchKernelGGL(k_patch_smooth<float>, dim3(g), dim3(256), 0, s, o, t, n, (long)nth, nphi);
         hipLaunchKernelGGL(k_patch_smooth<float>, dim3(g), dim3(256), 0, s, t, o, n, (long)nth * nphi, nr);

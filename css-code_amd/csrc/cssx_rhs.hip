@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "../../include/cssx.h"
+#include "cssx_bufio.hpp"
 #include "cssx_internal.hpp"
 #include "cssx_kernels.hpp"
 #include "cssx_plan.hpp"
@@ -981,7 +982,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 3 : 7) void k_rhs_final(Const
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_bound(Consts<T> c, BoundFlags f, const T *__restrict__ sr1, T *st, int nv) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long i = item_index();
     if (i >= c.N * nv) return;
     const int iv = (int)(i / c.N);
     const long j = i - (long)iv * c.N;
@@ -1046,7 +1047,7 @@ __global__ __launch_bounds__(256) void k_tvd_stage(Consts<TS> c, BoundFlags f, c
                                                    double *__restrict__ y0, double *__restrict__ ys,
                                                    const TS *__restrict__ k, const TS *__restrict__ dif,
                                                    TS *__restrict__ y1, int nv) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    long i = item_index();
     if (i >= c.N * nv) return;
     const int iv = (int)(i / c.N);
     const long j = i - (long)iv * c.N;
@@ -2041,7 +2042,6 @@ static int tvd_impl(cssx_mhd *m, double *y0, double dt, int nsteps, int order, h
     const Consts<T> c = make_consts<T>(m);
     const BoundFlags f = make_bound_flags(m);
     const long NV = m->N * m->nv;
-    const unsigned nb = nblocks(NV, 256);
     constexpr bool f32 = sizeof(T) != sizeof(double);
     T *dif = m->p.sld_on ? S.dif : nullptr;
     const double ts = (double)sizeof(T);
@@ -2049,7 +2049,7 @@ static int tvd_impl(cssx_mhd *m, double *y0, double dt, int nsteps, int order, h
         const double by = (ts + 8.0 + (mode ? 8.0 : 0.0) + (last && dif ? ts : 0.0) +
                            (last ? 8.0 + (f32 ? ts : 0.0) : 8.0 + ts)) * (double)NV;
         CSSX_TIMED(CSSX_PHASE_RK_UPDATE, stream, by,
-                   hipLaunchKernelGGL(k_tvd_stage<T>, dim3(nb), dim3(256), 0, stream, c, f,
+                   hipLaunchKernelGGL(k_tvd_stage<T>, item_grid(NV), dim3(256), 0, stream, c, f,
                                       (const double *)m->p64.sr1, (const double *)m->p64.rbar,
                                       (const double *)m->p64.sbar, mode, a0, a1, dtc, dt, last, y0, m->save,
                                       (const T *)S.k, (const T *)dif, S.y1, m->nv));
@@ -2236,10 +2236,10 @@ extern "C" int cssx_bound(cssx_mhd *m, int prec, void *state, void *stream) {
     const long NV = m->N * m->nv;
     const BoundFlags f = make_bound_flags(m);
     if (prec == CSSX_PREC_F64)
-        hipLaunchKernelGGL(k_bound<double>, dim3(nblocks(NV, 256)), dim3(256), 0, (hipStream_t)stream,
+        hipLaunchKernelGGL(k_bound<double>, item_grid(NV), dim3(256), 0, (hipStream_t)stream,
                            make_consts<double>(m), f, (const double *)m->p64.sr1, (double *)state, m->nv);
     else if (prec == CSSX_PREC_F32)
-        hipLaunchKernelGGL(k_bound<float>, dim3(nblocks(NV, 256)), dim3(256), 0, (hipStream_t)stream,
+        hipLaunchKernelGGL(k_bound<float>, item_grid(NV), dim3(256), 0, (hipStream_t)stream,
                            make_consts<float>(m), f, (const float *)m->p32.sr1, (float *)state, m->nv);
     else
         return CSSX_EINVAL;
