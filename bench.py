@@ -18,9 +18,11 @@ reported beside it.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import math
 import os
+import re
 import sys
 import time
 
@@ -38,6 +40,8 @@ HBM_PEAK_GBS = 8000.0
 # refreshes the FP32 copy): per field 12 + 20 + 20 + (4 + 4 + 8 + 8 + 4) = 80 B.
 STEP_BYTES_F64 = 1088.0
 STEP_BYTES_MIXED = 640.0
+# the kernel sources that no MHD step runs (step_sources)
+NOT_IN_A_STEP = ("cssx_closure.hip", "cssx_train.hpp", "cssx_patches.hip", "cssx_timing.hip")
 
 
 def _sync():
@@ -264,7 +268,7 @@ def run_c5(args):
 def run_c3(args):
     """Batched uneven derivatives: patches with every axis length uniform in [32, 512] (seed 4),
     FP32 N(0,1) smoothed by [1,2,1]/4 per axis, all three first derivatives of a chunk of patches
-    in one persistent launch (variant autotuned on the first chunk), chunks run back to back;
+    in one launch (variant autotuned on the first chunk), chunks run back to back;
     then the 64-member ensemble of 48x96x96 MHD runs (Ra log-uniform in [1e4, 1e6]) stepped
     eagerly and as one captured HIP graph."""
     import numpy as np
@@ -368,10 +372,31 @@ def run_deriv(args):
                                                       "nth": nth, "nphi": nphi}, "sweeps": res}))
 
 
-def measured_traffic(workload):
-    """The rocprofv3 FETCH_SIZE/WRITE_SIZE summary committed for this workload (FP32-bulk path):
-    the JSON block of profiles/hbm_traffic_<workload>.md, or None."""
-    path = os.path.join(ROOT, "profiles", f"hbm_traffic_{workload}.md")
+def step_sources():
+    """Fingerprint of the sources that an RK4 step's kernels and launches are built from, comments and white space
+    left out: a traffic profile holds for the kernels it was counted with."""
+    csrc = os.path.join(ROOT, "css-code_amd", "csrc")
+    h = hashlib.sha256()
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".hip", ".hpp", ".cpp")) or name in NOT_IN_A_STEP:
+            continue
+        with open(os.path.join(csrc, name)) as f:
+            text = re.sub(r"//[^\n]*|/\*.*?\*/", " ", f.read(), flags=re.S)
+        h.update((name + "\n" + " ".join(text.split()) + "\n").encode())
+    return h.hexdigest()[:16]
+
+
+def final_kernel(nth, precision, explicit_diffusion):
+    """The kernel that ends a right-hand side: k_rhs_line where it solves the theta derivatives itself (line_plan in
+    csrc/cssx_rhs.hip), else k_rhs_final."""
+    line = nth >= 32 if precision == "f32" else nth >= 48 and nth % 4 == 0
+    return "k_rhs_line" if line and not explicit_diffusion else "k_rhs_final"
+
+
+def measured_traffic(workload, folder=os.path.join(ROOT, "profiles")):
+    """The rocprofv3 FETCH_SIZE/WRITE_SIZE summary committed for this workload (FP32-bulk path): the JSON block of
+    profiles/hbm_traffic_<workload>.md, or None if there is none or it was counted with other kernels."""
+    path = os.path.join(folder, f"hbm_traffic_{workload}.md")
     if not os.path.exists(path):
         return None
     text = open(path).read()
@@ -382,6 +407,9 @@ def measured_traffic(workload):
     try:
         d = json.loads(text[i + 7:j])
     except ValueError:
+        return None
+    if d.get("step_sources") != step_sources():
+        print(f"bench: {os.path.basename(path)} was counted with other kernels: not used", file=sys.stderr, flush=True)
         return None
     d["source"] = os.path.relpath(path, ROOT)
     return d
@@ -537,12 +565,13 @@ def run_mhd(args, shape, seeds, study_steps, full):
     tab32 = profile_phases(sol, y0, dt, prof_steps, "f32") if "f32" in paths else None
     tab64 = profile_phases(sol, y0, dt, prof_steps, "f64") if ("f64" in paths and full) else None
 
-    families = {"k_deriv": ("deriv_r", "deriv_theta", "deriv_phi"), "k_rhs_final": ("rhs_final",),
+    def families(precision):
+        return {"k_deriv": ("deriv_r", "deriv_theta", "deriv_phi"), final_kernel(c.nth, precision, lap): ("rhs_final",),
                 "k_sld": ("sld",), "pointwise_other": ("pointwise",), "rk_stage": ("rk_update",)}
 
-    def family_rows(tab):
+    def family_rows(tab, precision):
         rows = {}
-        for name, ph in families.items():
+        for name, ph in families(precision).items():
             ms = sum(tab[k][0] for k in ph)
             n = sum(tab[k][1] for k in ph)
             by = sum(tab[k][2] for k in ph)
@@ -553,14 +582,14 @@ def run_mhd(args, shape, seeds, study_steps, full):
                               "achieved_GBs": round(ach, 1), "frac": round(ach / HBM_PEAK_GBS, 4)}
         return rows
 
-    def roofline(tab):
+    def roofline(tab, precision):
         """Roofline of the dominant kernel family (largest summed time): achieved = algorithmic
         bytes per launch / average launch time, both from the per-launch hipEvent timer."""
         if tab is None:
             return None
-        rows = family_rows(tab)
+        rows = family_rows(tab, precision)
         name = max(rows, key=lambda k: rows[k]["ms_per_step"])
-        ph = families[name]
+        ph = families(precision)[name]
         ms = sum(tab[k][0] for k in ph)
         n = sum(tab[k][1] for k in ph)
         by = sum(tab[k][2] for k in ph)
@@ -574,7 +603,7 @@ def run_mhd(args, shape, seeds, study_steps, full):
     val32 = npts / (ms32 * 1e-3) / 1e6
     val64 = npts / (ms64 * 1e-3) / 1e6
     tr = measured_traffic(workload)
-    roof32 = roofline(tab32)
+    roof32 = roofline(tab32, "f32")
     if roof32 is not None and tr is not None and roof32["kernel"] in tr.get("families", {}):
         roof32["traffic"] = tr["families"][roof32["kernel"]]["bytes_per_launch"]
         roof32["traffic_source"] = tr["source"]
@@ -610,10 +639,10 @@ def run_mhd(args, shape, seeds, study_steps, full):
         "roofline": roof32,
     }
     if full:
-        out["roofline_f64"] = roofline(tab64)
+        out["roofline_f64"] = roofline(tab64, "f64")
         out["phases_ms_per_step"] = {p: ({k: round(v[0] / prof_steps, 4) for k, v in t.items()} if t else None)
                                      for p, t in (("f32", tab32), ("f64", tab64))}
-        out["kernel_families"] = {p: (family_rows(t) if t else None) for p, t in (("f32", tab32), ("f64", tab64))}
+        out["kernel_families"] = {p: (family_rows(t, p) if t else None) for p, t in (("f32", tab32), ("f64", tab64))}
     sol.close()
     del y0
     torch.cuda.empty_cache()
