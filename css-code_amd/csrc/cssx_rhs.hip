@@ -4,8 +4,8 @@
 // Laplacian / SLaplacian explicit diffusion) is evaluated as:
 //   1. curl A: six batched derivative sweeps whose epilogues apply the metric factors and add
 //      the second term of each component onto the first (Compute_B, derivatives.f90:1830-1892)
-//   2. k_walls_state: Compute_B's wall conditions on the wall points, and the wall values of the closures that depend on the state (rhs_mpi.f90:410-455,
-//      :578-637)
+//   2. k_walls_state: Compute_B's wall conditions on the wall points, and the wall values of the
+//      closures that depend on the state (rhs_mpi.f90:410-455, :578-637)
 //   3. the 19 first-derivative sweeps of Source_Theta_Terms / Phi_Terms / Radial_Terms, batched
 //      per axis (one launch per axis, one job per field); with explicit diffusion also the 12
 //      second derivatives, the 6 cross-term sweeps of first-derivative slots and the 3 or 4
@@ -18,9 +18,9 @@
 //   6. two density sweeps + k_rhs_final: the terms of step 4 at every point, the density terms,
 //      top relaxation, u x B (and -etar curl B with its Ohmic heating), xi_cs and the fused RK4
 //      stage; no tendency field is written and re-read in between
-// Without explicit diffusion and for the theta sizes of line_plan, k_rhs_line takes the place of k_rhs_final, of
-// the theta sweeps of steps 3 and 6 and of the theta walls of step 5, and the density's r sweep runs with those of
-// step 3 (cssx_rhs_line.hpp).
+// Without explicit diffusion and for the theta sizes of line_plan, k_rhs_line takes the place of
+// k_rhs_final, of the theta sweeps of steps 3 and 6 and of the theta walls of step 5, and the
+// density's r sweep runs with those of step 3 (cssx_rhs_line.hpp).
 // Temperature T = rho^(gamma-1) exp(s/Cv)/((gamma-1)Cv) and 1/rho are recomputed where used
 // instead of being stored (rhs_mpi.f90:377-387).
 #include <hip/hip_runtime.h>

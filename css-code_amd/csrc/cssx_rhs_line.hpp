@@ -8,9 +8,10 @@
 // them.  The terms are those of main_terms and final_point, in their order, over the lane's points.
 //
 // Bound by memory: per stage the seven theta sweeps' 14 fields of traffic and the final kernel's 7
-// reads of them go away.  256x512x1024 FP32 RK4 stage: 6.95 ms of k_rhs_final + 1.30 of theta sweeps + 0.1 of
-// k_walls_gather -> 6.00 ms, now 5.73 (average of the four stages); 128x256x512 FP64: 1.63 + 0.42 -> 1.43, now 1.36.  Eight points per lane (512
-// rows in one wavefront, one wavefront per SIMD) took 8.53 ms, three wavefronts per SIMD (spills) 10.3 ms.
+// reads of them go away.  256x512x1024 FP32 RK4 stage: 6.95 ms of k_rhs_final + 1.30 of theta sweeps
+// + 0.1 of k_walls_gather -> 6.00 ms, now 5.68 (average of the four stages); 128x256x512 FP64:
+// 1.63 + 0.42 -> 1.43, now 1.36.  Eight points per lane (512 rows in one wavefront, one wavefront per
+// SIMD) took 8.53 ms, three wavefronts per SIMD (spills) 10.3 ms.
 #pragma once
 
 #include "cssx_line.hpp"
