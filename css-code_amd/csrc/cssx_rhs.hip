@@ -992,6 +992,12 @@ __global__ __launch_bounds__(256) void k_bound(Consts<T> c, BoundFlags f, const 
 }
 
 // ---------------------------------------------------------------------------------------------
+template <typename T>
+__global__ __launch_bounds__(256) void k_zero(T *__restrict__ p, long n) {
+    const long i = item_index();
+    if (i < n) p[i] = T(0);
+}
+
 // y1 = (float)(y0 - background) (first step of an FP32 run; rho and s as fluctuations): one row of workgroups per
 // (field, ir), so that the background is one scalar, eight values per thread as 16-byte accesses.
 // Bound by memory: 256x512x1024, 8 fields 3.24 -> 2.28 ms (4.0 -> 5.65 TB/s).
@@ -1360,6 +1366,10 @@ static int ensure_scratch(cssx_mhd *m) {
     if (hipMalloc(&S.y1, sizeof(T) * N * m->nv) != hipSuccess) return CSSX_ENOMEM;
     if (hipMalloc(&S.k, sizeof(T) * N * m->nv) != hipSuccess) return CSSX_ENOMEM;
     if (m->p.sld_on && hipMalloc(&S.dif, sizeof(T) * N * m->nv) != hipSuccess) return CSSX_ENOMEM;
+    // without Magnetic_Diffusion nothing ever writes A's SLD tendency, which the steps add all the same
+    if (m->p.sld_on && m->p.magnetic && !m->p.magnetic_diffusion &&
+        (hipMemset(S.dif + 5 * N, 0, sizeof(T) * N * 3) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess))
+        return CSSX_EHIP;
     if (m->p.sld_on && hipMalloc(&S.vcc, sizeof(T) * N) != hipSuccess) return CSSX_ENOMEM;
     {
         const size_t tw = (size_t)(8 + D_NSLOT) * 2 * m->nr * m->nphi;
@@ -2263,6 +2273,8 @@ static int diffusion_entry(cssx_mhd *m, const T *st, const T *b, T *dif, hipStre
         if ((rc = curl_impl<T>(m, st + 5 * m->N, S.B, stream))) return rc;
         B = S.B;
     }
+    if (m->p.magnetic && !m->p.magnetic_diffusion)   // A is not diffused
+        hipLaunchKernelGGL(k_zero<T>, item_grid(3 * m->N), dim3(256), 0, stream, dif + 5 * m->N, 3 * m->N);
     return sld_impl<T>(m, st, B, dif, stream);
 }
 
